@@ -17,6 +17,8 @@ struct GroupBufs {
     int32_t* meta;    // [4]: active experts, bad ids, passes of the work list, passes of the second list
     int32_t* items;   // pass list, room for max_passes(n, E, 16) (expert, pass, passes) triples
     int32_t* items2;  // second pass list (dense down after wave gate/up), room for max_passes(n, E, 64)
+    int32_t* chunks;  // scratch of the two-launch grouping (per-chunk counts), or null: one workgroup groups the slots
+    size_t chunks_n;  // its room in ints
 };
 
 // One router launch (moe_router.hip): the logits, then (tail) the top-k tail per token, the merged slot lists with
@@ -57,10 +59,9 @@ int launch_router_logits(const uint16_t* x, const uint16_t* wr, const float* bia
 // lstride: elements between logit rows (0: E)
 int launch_topk(const void* logits, int dtype, int T, int E, int k, int norm, float scale, int32_t* idx, float* wts,
                 hipStream_t st, int lstride = 0);
-// with items: also the grouped kernels' pass list for passes of P slots (items [3 * max_passes(n, E, P)], meta[2])
-int launch_group(const int32_t* idx, int n, int E, int32_t* counts, int32_t* offsets, int32_t* sorted,
-                 int32_t* active, int32_t* meta, hipStream_t st, int P = 0, int32_t* items = nullptr, int P2 = 0,
-                 int32_t* items2 = nullptr);
+// stable grouping of the ids idx[n] into o (with o.items / o.items2 also the grouped kernels' pass lists, passes of P and
+// P2 slots); with o.chunks and many slots in two launches, else in one workgroup
+int launch_group(const int32_t* idx, int n, int E, const GroupBufs& o, hipStream_t st, int P = 0, int P2 = 0);
 // tuning and test knobs from the environment, read per call
 inline int env_int(const char* name, int dflt) {
     const char* v = getenv(name);

@@ -182,6 +182,70 @@ __global__ void __launch_bounds__(64 * FIN_WAVES) route_finish(RouterArgs a) {
     group_block([&](int p) { return load_agent(ids + p); }, n, Eg, a.grp, a.P, a.P2, sm, a.mw);
 }
 
+// The same for calls with many slots (two-launch grouping, moe_group.h): SPLIT_WAVES tokens at a time, one per wave,
+// tok tokens per workgroup (a chunk), whose slots are counted per expert in LDS and written to a.grp.chunks[workgroup].
+// Every SIMD runs four tails at once here (they are VALU-issue bound), where route_finish spreads few tails over many
+// CUs.
+constexpr int SPLIT_WAVES = 16;
+template <int JM>
+__global__ void __launch_bounds__(64 * SPLIT_WAVES) route_tails(RouterArgs a, int tok) {
+    extern __shared__ int32_t sm[];   // counts [E + S]
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int k = a.k, ws = a.k + a.S, Eg = a.E + a.S;
+    int32_t* ids = a.S ? a.sidx : a.idx;
+    const int t0 = blockIdx.x * tok, t1 = t0 + tok < a.T ? t0 + tok : a.T;
+    for (int i = threadIdx.x; i < Eg; i += 64 * SPLIT_WAVES) sm[i] = 0;
+    __syncthreads();
+    for (int t = t0 + wave; t < t1; t += SPLIT_WAVES) {
+        const float* lrow = a.logits + (size_t)t * a.lstride;
+        float v[JM];
+#pragma unroll
+        for (int j = 0; j < JM; ++j) v[j] = j * 64 + lane < a.E ? lrow[j * 64 + lane] : -INFINITY;
+        const float gl = a.gate ? lrow[a.E] : 0.f;
+        uint32_t id;
+        float w;
+        topk_core<JM>(v, a.E, k, a.norm, a.scale, k, &id, &w);
+        int32_t sid = (int32_t)id;
+        if (a.S && lane >= k) sid = a.E + lane - k;
+        if (lane < k) {
+            if (a.S) a.idx[(size_t)t * k + lane] = sid;
+            a.wts[(size_t)t * k + lane] = w;
+        }
+        if (lane < ws) {
+            if (a.S) a.swts[(size_t)t * ws + lane] = lane < k ? w : (a.gate ? 1.f / (1.f + expf(-gl)) : 1.f);
+            ids[(size_t)t * ws + lane] = sid;
+            atomicAdd(&sm[sid], 1);
+        }
+    }
+    if (a.xterm) {   // x's fp8 term records, as in route_finish
+        const int nsl = (a.d + 127) >> 7;
+        for (int i = threadIdx.x; i < (t1 - t0) * 4 * nsl; i += 64 * SPLIT_WAVES)
+            mx_terms_block<2>(a.x + (size_t)t0 * a.d, t1 - t0, a.d, a.xterm + (size_t)t0 * nsl * mx_rec<2>(), i);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < Eg; i += 64 * SPLIT_WAVES) a.grp.chunks[(size_t)blockIdx.x * Eg + i] = sm[i];
+}
+
+// Two-launch grouping of given ids: the counts of each chunk of cs slots, then the placing workgroups.
+__global__ void __launch_bounds__(256) k_group_count(const int32_t* __restrict__ idx, int n, int E, int cs,
+                                                     int32_t* __restrict__ chunks) {
+    extern __shared__ int32_t sm[];
+    const int b0 = blockIdx.x * cs, b1 = b0 + cs < n ? b0 + cs : n;
+    for (int i = threadIdx.x; i < E; i += 256) sm[i] = 0;
+    __syncthreads();
+    for (int p = b0 + threadIdx.x; p < b1; p += 256) {
+        const int e = idx[p];
+        if (e >= 0 && e < E) atomicAdd(&sm[e], 1);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < E; i += 256) chunks[(size_t)blockIdx.x * E + i] = sm[i];
+}
+__global__ void __launch_bounds__(1024) k_group_place(const int32_t* __restrict__ idx, int n, int E, int cs, int nchunk,
+                                                      GroupBufs o, int P, int P2) {
+    extern __shared__ int32_t sm[];
+    group_place(idx, n, E, cs, nchunk, o, P, P2, sm);
+}
+
 // Router tail on given logits [T, E] (fp32, bf16 or fp16): one wave per token.
 template <typename LT>
 __global__ void __launch_bounds__(256)
@@ -260,6 +324,17 @@ shared_route(const void* __restrict__ x, int xdt, const uint16_t* __restrict__ g
 // per-wave count arrays up to FIN_LDS, else the counts and cursors only, with wave 0 placing every slot.
 constexpr size_t FIN_LDS = 32 * 1024;
 
+// whether a call's grouping is split over chunks (two launches): enough slots, and scratch for the count rows
+static bool group_split(int n, int E, int nchunk, const GroupBufs& o) {
+    return o.chunks && n >= env_int("MOE_GROUP_SPLIT_MIN", GROUP_SPLIT_MIN) && E <= GROUP_SPLIT_MAX_E &&
+           (size_t)nchunk * E <= o.chunks_n;
+}
+static int launch_group_place(const int32_t* idx, int n, int E, int cs, int nchunk, const GroupBufs& o, int P, int P2,
+                              hipStream_t st) {
+    k_group_place<<<nchunk + 1, 1024, (size_t)group_place_lds_ints(E) * 4, st>>>(idx, n, E, cs, nchunk, o, P, P2);
+    return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
+}
+
 // logits (T > 1: ROUTER_TPW tokens per wave share each loaded Wr chunk; T == 1: one expert per wave, fewer larger
 // waves or one wave per workgroup spread over E CUs measured no faster)
 int launch_route_logits(const RouterArgs& a, hipStream_t st) {
@@ -275,8 +350,21 @@ int launch_route(RouterArgs a, bool tail, hipStream_t st) {
     if (a.grp.counts && ((a.grp.items && (a.P < 1 || (a.P & (a.P - 1)))) ||
                          (a.grp.items2 && (a.P2 < 1 || (a.P2 & (a.P2 - 1))))))
         return MOE_ERR_ARG;   // pass sizes are powers of two
+    const int n_all = a.T * (a.k + a.S), E_all = a.E + a.S;
+    const int tok = group_chunk(a.T, SPLIT_WAVES), nchunk = (a.T + tok - 1) / tok;
+    const bool split = tail && a.grp.counts && group_split(n_all, E_all, nchunk, a.grp);
+    if (split) a.arrive = nullptr;
     int rc = launch_route_logits(a, st);
     if (rc || !tail) return rc;
+    if (split) {
+        const size_t lds = (size_t)E_all * 4;
+        if (a.E <= 64) route_tails<1><<<nchunk, 64 * SPLIT_WAVES, lds, st>>>(a, tok);
+        else if (a.E <= 128) route_tails<2><<<nchunk, 64 * SPLIT_WAVES, lds, st>>>(a, tok);
+        else if (a.E <= 256) route_tails<4><<<nchunk, 64 * SPLIT_WAVES, lds, st>>>(a, tok);
+        else route_tails<TOPK_MAX_J><<<nchunk, 64 * SPLIT_WAVES, lds, st>>>(a, tok);
+        if (hipGetLastError() != hipSuccess) return MOE_ERR_LAUNCH;
+        return launch_group_place(a.S ? a.sidx : a.idx, n_all, E_all, tok * (a.k + a.S), nchunk, a.grp, a.P, a.P2, st);
+    }
     size_t lds = 0;
     if (a.grp.counts) {
         const int n = a.T * (a.k + a.S), Eg = a.E + a.S;
@@ -330,15 +418,19 @@ int launch_shared_route(const void* x, int xdt, const uint16_t* gate, int T, int
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
-int launch_group(const int32_t* idx, int n, int E, int32_t* counts, int32_t* offsets, int32_t* sorted,
-                 int32_t* active, int32_t* meta, hipStream_t st, int P, int32_t* items, int P2, int32_t* items2) {
-    if ((items && (P < 1 || (P & (P - 1)))) || (items2 && (P2 < 1 || (P2 & (P2 - 1))))) return MOE_ERR_ARG;
+int launch_group(const int32_t* idx, int n, int E, const GroupBufs& o, hipStream_t st, int P, int P2) {
+    if ((o.items && (P < 1 || (P & (P - 1)))) || (o.items2 && (P2 < 1 || (P2 & (P2 - 1))))) return MOE_ERR_ARG;
+    const int cs = group_chunk(n, 128), nchunk = (n + cs - 1) / cs;
+    if (group_split(n, E, nchunk, o)) {
+        k_group_count<<<nchunk, 256, (size_t)E * 4, st>>>(idx, n, E, cs, o.chunks);
+        if (hipGetLastError() != hipSuccess) return MOE_ERR_LAUNCH;
+        return launch_group_place(idx, n, E, cs, nchunk, o, P, P2, st);
+    }
     // one block: 16 waves (1024 threads) each placing a sixteenth of the slots from 1024 slots, else 4 waves; the
     // per-wave counts and the ids in LDS (at most 64 KB), else wave 0 places all of them
     int nw = n >= 1024 ? 16 : 4;
     if ((size_t)group_lds_ints(n, E, nw, 1) * 4 > 64 * 1024) nw = 4;
     const int mw = (size_t)group_lds_ints(n, E, nw, 1) * 4 <= 64 * 1024 ? 1 : 0;
-    const GroupBufs o{counts, offsets, sorted, active, meta, items, items2};
     group_slots<<<1, 64 * nw, (size_t)group_lds_ints(n, E, nw, mw) * 4, st>>>(idx, n, E, o, P, P2, mw);
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }

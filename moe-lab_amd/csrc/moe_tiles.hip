@@ -2102,11 +2102,9 @@ int run_tiles_fmt(const ExpertsArgs& a) {
         if (t.eslot_off + (size_t)nslots * 4 > (size_t)nslots * w->F * 2) return MOE_ERR_ARG;
     }
     if (a.stages & 1) {
-        int rc = ingroup || a.pregrouped
-                     ? 0
-                     : launch_group(a.idx, nslots, w->E, a.grp.counts, a.grp.offsets, a.grp.sorted, a.grp.active,
-                                       a.grp.meta, a.st, P_gu, a.grp.items, two_lists ? P_dn : 0,
-                                       two_lists ? a.grp.items2 : nullptr);
+        GroupBufs grp = a.grp;
+        if (!two_lists) grp.items2 = nullptr;
+        int rc = ingroup || a.pregrouped ? 0 : launch_group(a.idx, nslots, w->E, grp, a.st, P_gu, P_dn);
         if (rc) return rc;
         TileArgs g = t;
         if (emit) {
