@@ -1,7 +1,7 @@
 // Router and slot grouping kernels for gfx950.
 //
-// router_logits: logits[t, e] = x[t] . Wr[e] (+ b[e]) in fp32, one wave per EPW experts x TPW tokens. route_finish,
-// the next launch: the router tail (top-k, softmax) of one token per wave and, when the call asks for the grouping,
+// router_logits: logits[t, e] = x[t] . Wr[e] (+ b[e]) in fp32, one wave per EPW experts x TPW tokens (router_logits_mm:
+// the same on the fp32 matrix cores for many tokens). route_finish, the next launch: the router tail (top-k, softmax) of one token per wave and, when the call asks for the grouping,
 // the sort of all T*k slots by expert (group_block) in its last workgroup to finish. At T = 1 the layer call skips
 // route_finish: the gate/up waves rank the token's logits themselves (moe_experts.hip).
 // The logit reduction order is fixed, so a CPU restatement reproduces every logit bit for bit and top-k ids
@@ -37,6 +37,12 @@ __device__ __forceinline__ float to_f32<uint16_t>(uint16_t v) { return bf16_to_f
 template <>
 __device__ __forceinline__ float to_f32<_Float16>(_Float16 v) { return (float)v; }
 
+// logits (tokens x rows) from which they run on the matrix cores (router_logits_mm): its launch costs a fixed ~3 us more
+// (row gathers, the rank-1 MFMA chain), the vector form's time grows with tokens x rows. Logits + tails, vector / matrix:
+// E = 128 T = 128 7.6 / 8.9 us, T = 256 10.3 / 9.0; E = 64 T = 256 7.8 / 8.8, T = 512 10.5 / 9.0; E = 32 d = 2880 T = 512
+// 10.0 / 11.9, T = 1500 22 / 12.8; E = 8 d = 4096 T = 1500 9.9 / 12.1, T = 4096 19.4 / 14.0; E = 256 d = 7168 T = 96
+// 21.5 / 21.1, T = 256 46 / 21.5
+constexpr int ROUTER_MM_MIN = 24576;
 constexpr int ROUTER_MAXC = 4;   // 16-byte chunks per lane held in registers per pass (2048 inputs)
 
 // Logits: grid (ceil(rows / (ROUTER_WAVES * EPW)), ceil(T / TPW)), block 64 * ROUTER_WAVES; rows = a.lstride (the E
@@ -109,6 +115,100 @@ __global__ void __launch_bounds__(64 * ROUTER_WAVES) router_logits(RouterArgs a)
                 a.logits[(size_t)(t0 + i) * rows + e] = s;
             }
         }
+}
+
+// Logits of many tokens on the matrix cores, in the same order bit for bit. v_mfma_f32_16x16x1_4b_f32 is a rank-1 update
+// of four independent 16 x 16 blocks, one fused multiply-add per output in fp32 (checked bit for bit against fmaf,
+// subnormals included), so a block per virtual lane l gives the lane partials a[l] of every (token, row) of a tile: A
+// holds element i of chunk l, l + 64, ... of 16 tokens, B the same element of 16 router rows. The DPP tree of
+// sum_lanes<64> over the lanes then is plain adds of accumulator registers.
+// A workgroup owns 16 TT tokens x 16 rows; wave w of 8 takes the lanes 8 w .. 8 w + 7 (their chunks are 128 contiguous
+// bytes per row) and leaves H[w] in LDS. d % 64 == 0, so a wave's eight lanes always have equally many chunks. The
+// loads of MB chunks go out together: with a chunk or two in flight the latency of the row gathers is what it costs.
+// Bound: the fp32 MFMA rate (twice the FMA rate of the vector pipe) and the L2 reads of x, once per 16 rows; the vector
+// form re-reads x once per row and unpacks bf16 per product. Workgroups are numbered so that the row blocks of a
+// token block share an XCD (x stays in its L2). Qwen3 T = 4096 (E = 128, d = 2048),
+// logits and tails: 88 -> 32 us.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+template <int TT, int MB>
+__global__ void __launch_bounds__(512) router_logits_mm(RouterArgs a) {
+    __shared__ float sH[8][TT][256];
+    const int rows = a.lstride, d = a.d, nchunk = d >> 3;
+    const int nrb = (rows + 15) >> 4, ntb = (a.T + 16 * TT - 1) / (16 * TT);
+    if (a.arrive && blockIdx.x == 0 && threadIdx.x == 0) *a.arrive = 0;
+    const int b8 = (int)(blockIdx.x >> 3), rb = b8 % nrb, tb = (int)(blockIdx.x & 7) + 8 * (b8 / nrb);
+    if (tb >= ntb) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int r = lane & 15, blk = lane >> 4;
+    const int e = min(16 * rb + r, rows - 1);
+    const uint4* wp = reinterpret_cast<const uint4*>(e < a.E ? a.wr + (size_t)e * d : a.gate) + blk;
+    const uint4* xp[TT];
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+        xp[i] = reinterpret_cast<const uint4*>(a.x + (size_t)min(16 * (TT * tb + i) + r, a.T - 1) * d) + blk;
+    f32x16 acc[2][TT];   // lanes 8 w + 4 q .. + 3: block b of the MFMA is lane 8 w + 4 q + b
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int i = 0; i < TT; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[q][i][v] = 0.f;
+    const int c0 = 8 * wave, nm = c0 < nchunk ? (nchunk - c0 + 63) >> 6 : 0;
+    for (int m0 = 0; m0 < nm; m0 += MB) {
+        uint4 w[MB][2], xv[MB][2][TT];
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            const int c = c0 + 64 * (m0 + m < nm ? m0 + m : nm - 1);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                w[m][q] = wp[c + 4 * q];
+#pragma unroll
+                for (int i = 0; i < TT; ++i) xv[m][q][i] = xp[i][c + 4 * q];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+            if (m0 + m < nm) {   // wave-uniform
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {   // element u of the chunks
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const uint4& wr = w[m][q];
+                        const uint32_t ww = (u >> 1) == 0 ? wr.x : ((u >> 1) == 1 ? wr.y : ((u >> 1) == 2 ? wr.z : wr.w));
+                        const float wf = u & 1 ? bf16hi(ww) : bf16lo(ww);
+#pragma unroll
+                        for (int i = 0; i < TT; ++i) {
+                            const uint4& xr = xv[m][q][i];
+                            const uint32_t xw = (u >> 1) == 0 ? xr.x : ((u >> 1) == 1 ? xr.y : ((u >> 1) == 2 ? xr.z : xr.w));
+                            acc[q][i] = __builtin_amdgcn_mfma_f32_16x16x1f32(u & 1 ? bf16hi(xw) : bf16lo(xw), wf, acc[q][i], 0, 0, 0);
+                        }
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            float Q[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                Q[q] = (acc[q][i][v] + acc[q][i][4 + v]) + (acc[q][i][8 + v] + acc[q][i][12 + v]);
+            sH[wave][i][(4 * blk + v) * 16 + r] = Q[0] + Q[1];
+        }
+    __syncthreads();
+    for (int o = threadIdx.x; o < 256 * TT; o += 512) {
+        const int i = o >> 8, p = o & 255, t = 16 * (TT * tb + i) + (p >> 4), er = 16 * rb + (p & 15);
+        const float R0 = sH[0][i][p] + sH[1][i][p], R1 = sH[2][i][p] + sH[3][i][p], R2 = sH[4][i][p] + sH[5][i][p],
+                    R3 = sH[6][i][p] + sH[7][i][p];
+        float s = (R3 + R2) + (R1 + R0);
+        if (t < a.T && er < rows) {
+            if (a.bias && er < a.E) s = s + a.bias[er];
+            a.logits[(size_t)t * rows + er] = s;
+        }
+    }
 }
 
 // The rest of the router, on the logits of the previous launch (its kernel boundary makes them visible): one wave per
@@ -335,9 +435,17 @@ static int launch_group_place(const int32_t* idx, int n, int E, int cs, int nchu
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
-// logits (T > 1: ROUTER_TPW tokens per wave share each loaded Wr chunk; T == 1: one expert per wave, fewer larger
+// logits (T > 1, fewer than ROUTER_MM_MIN logits: ROUTER_TPW tokens per wave share each loaded Wr chunk; T == 1: one expert per wave, fewer larger
 // waves or one wave per workgroup spread over E CUs measured no faster)
 int launch_route_logits(const RouterArgs& a, hipStream_t st) {
+    if ((long)a.T * a.lstride >= env_int("MOE_ROUTER_MM_MIN", ROUTER_MM_MIN) && a.d % 64 == 0) {
+        const int nrb = (a.lstride + 15) / 16, n2 = (a.T + 31) / 32, n1 = (a.T + 15) / 16;
+        const bool two = (long)n2 * nrb >= 512;   // two token tiles per wave (w read half as often) once they fill the chip
+        const unsigned grid = 8u * nrb * (((two ? n2 : n1) + 7) / 8);
+        if (two) router_logits_mm<2, 2><<<grid, 512, 0, st>>>(a);
+        else router_logits_mm<1, 4><<<grid, 512, 0, st>>>(a);
+        return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
+    }
     const dim3 grid((a.lstride + ROUTER_WAVES - 1) / ROUTER_WAVES, a.T == 1 ? 1 : (a.T + ROUTER_TPW - 1) / ROUTER_TPW);
     if (a.T == 1) router_logits<1, 1><<<grid, 64 * ROUTER_WAVES, 0, st>>>(a);
     else router_logits<ROUTER_TPW, 1><<<grid, 64 * ROUTER_WAVES, 0, st>>>(a);
