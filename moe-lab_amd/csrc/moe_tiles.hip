@@ -57,7 +57,6 @@ __device__ __forceinline__ int h16_exponent(float amax) {
     return 0;
 }
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int TL_ROWS = 64;   // weight rows per block
 constexpr int TL_KC = 8;      // chunks (32 inputs) per K slice
 constexpr int TL_APAD = 4 * TL_KC + 4;   // words per staged row: [g 0..3][chunk 0..KC-1] + 4 words of padding
@@ -961,92 +960,68 @@ __global__ void __launch_bounds__(64) k_wave_tile(TileArgs a) {
 
 // ============================================================================ dense tiles (many tokens per expert)
 // Where an expert's token count makes the contraction dense (tens to hundreds of tokens per expert: prefill, the
-// shared experts), each block keeps its weight tiles for a pass of 64 tokens and multiplies them on MFMA
-// against activations staged once per block in LDS. k_dense: a block of 4 waves owns BN rows of one expert (gate
-// and up: 128 rows of each, the GLU applied in registers; down: 256 rows) and one pass of the work list (up to
-// 16 * NT tokens of it); each wave covers all the pass's tokens for its 64 rows. (8-wave blocks of 128 tokens,
-// sharing each weight tile between two token halves, measured slower: one barrier domain per CU instead of two
-// independent blocks.) Per K slice of 128 inputs:
-//   activations: the pass's token rows, brought into LDS by global_load_lds_dwordx4 (16 bytes per lane, 4 token
-//     rows of 256 bytes per instruction); piece p (8 inputs) of token m lies at position p ^ (m & 15) of the
-//     token's row, so the MFMA operand reads (16 tokens x one piece) hit distinct banks. Two buffers (distinct
-//     objects, so the compiler's LDS-DMA tracking sees that a read of one does not wait for the DMA into the
-//     other): slice s + 1 is in flight while slice s is multiplied; one vmcnt(0) + barrier per slice.
-//   weights: each wave streams its own 16-row tiles from the tile-major records (1 KB code burst + metadata per
-//     tile and slice) into registers one slice ahead and decodes them exactly (int4: bf16 128 + q; MXFP4:
-//     e2m1(q)), in natural order (the records interleave each word's nibbles for that).
-//   product: token-major like the wave tiles, D[token, row] on v_mfma_f32_16x16x32_bf16 (activations A, codes
-//     B) with the same per-group fp32 fold: per scale group P = sum code * x, int4 XS = sum x (one MFMA with an
-//     all-ones operand per token tile), acc += s P + (b - 128 s) XS, or acc += 2^(e-127) P.
-// Rounding the dequantised weights to bf16 instead would put up to ~2% of RMS of error on the outputs, and h
-// kept in one bf16 plane (the reference keeps h in x.dtype) ~1%; the exact operands and h as two bf16 planes
-// h = hi + lo (natural order, the wave tiles' layout) keep the error to fp32 accumulation. Down runs one MFMA
-// per plane into the same accumulator and writes yp[slot] in fp32 for k_combine.
+// shared experts), each block keeps its weight tiles for a pass of 64 tokens and multiplies them on MFMA against
+// activations staged once per block in LDS: k_dense_i4 (int4, moe_dense_i4.h), k_mxd (MXFP4 with bf16 x) and k_dense
+// (MXFP4 with fp16 / fp32 x, or MOE_MXMFMA=0: exact codes on bf16 MFMA).
 #define MOE_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
 // s_waitcnt vmcnt(0) with the other counters left alone (gfx9 encoding)
 #define MOE_VMWAIT0() __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8))
 // workgroup barrier without a memory fence; the "memory" clobber keeps LDS accesses on their side of it
 #define MOE_BARRIER() asm volatile("s_barrier" ::: "memory")
 
-// Dense tile shapes (measured at the Mixtral T=512 shape). int4 down (operands decoded to fp16 with the scale
-// applied, no fold): 32 rows per wave; dense_nt's 128-token passes (each decoded operand feeding 8 MFMAs, 64
-// accumulators, 2 waves per SIMD) measured 234 -> 214 us in the kernel alone against 64-token passes, but the call
-// runs 64-token passes (make_plan's dn_nt): 4 waves per SIMD and no K split, faster per layer. int4 gate/up keeps
-// 64-token passes with 32 rows of each
-// projection per wave: with 128 tokens and 16 rows each, every activation slice staged in LDS serves half as many
-// rows (K = d is long, the L2 -> LDS traffic doubles) and the kernel slowed 440 -> 509 us. MXFP4 (raw codes on
-// bf16 MFMA, fp32 fold per group): 64-token passes, 32 / 64 rows per wave.
-// The dense tiles' passes of one expert split its ceil(n / 16) token tiles evenly: pass p of np takes tiles
-// [p T / np, (p + 1) T / np), at most ceil(T / np) <= BM / 16 of them. Passes that share a weight tile then do
-// the same MFMA work and stream the tile side by side on one XCD (a short tail pass would run ahead of its
-// partner, and the partner's weight reads would miss the L2).
+// The dense tiles' passes of one expert split its ceil(n / M) token tiles evenly: pass p of np takes tiles
+// [p T / np, (p + 1) T / np), at most ceil(T / np) of them. Passes that share a weight tile then do the same MFMA work
+// and stream the tile side by side on one XCD (a short tail pass would run ahead of its partner, and the partner's
+// weight reads would miss the L2).
+template <int M = 16>
 __device__ __forceinline__ void pass_tokens(int n, int np, int p, int& tok0, int& nlive) {
-    const int nt = (n + 15) >> 4;
+    const int nt = (n + M - 1) / M;
     const int t0 = p * nt / np, t1 = (p + 1) * nt / np;
-    tok0 = 16 * t0;
-    nlive = (16 * t1 < n ? 16 * t1 : n) - tok0;
+    tok0 = M * t0;
+    nlive = (M * t1 < n ? M * t1 : n) - tok0;
 }
 
+// k_dense: a block of 4 waves owns 256 / NPROJ rows of one expert (per projection) and one pass of up to 64 of its
+// tokens; each wave covers all the pass's tokens for its rows. Per K slice of 128 inputs:
+//   activations: the pass's token rows, brought into LDS by global_load_lds_dwordx4 (16 bytes per lane, 4 token
+//     rows of 256 bytes per instruction); piece p (8 inputs) of token m lies at position p ^ (m & 15) of the
+//     token's row, so the MFMA operand reads (16 tokens x one piece) hit distinct banks. Two buffers (distinct
+//     objects, so the compiler's LDS-DMA tracking sees that a read of one does not wait for the DMA into the
+//     other): slice s + 1 is in flight while slice s is multiplied; one vmcnt(0) + barrier per slice.
+//   weights: each wave streams its own 16-row tiles from the tile-major records (1 KB code burst + metadata per
+//     tile and slice) into registers one slice ahead and decodes them exactly (e2m1(q)), in natural order (the
+//     records interleave each word's nibbles for that).
+//   product: token-major like the wave tiles, D[token, row] on v_mfma_f32_16x16x32_bf16 (activations A, codes B); per
+//     32-input scale group P = sum code * x, then acc += 2^(e-127) P in fp32.
+// h is kept as two bf16 planes h = hi + lo (natural order, the wave tiles' layout); down runs one MFMA per plane into
+// the same accumulator and writes yp[slot] in fp32 for k_combine.
+template <int NPROJ>
+__host__ __device__ constexpr int dense_mx_rt() { return 4 / NPROJ; }   // 16-row tiles per projection per wave
 template <class FMT, int NPROJ>
-__host__ __device__ constexpr int dense_nt() { return FMT::XSUM && NPROJ == 1 ? 8 : 4; }
-template <class FMT, int NPROJ>
-__host__ __device__ constexpr int dense_rt() { return FMT::XSUM ? 2 : 4 / NPROJ; }
-template <class FMT, int NPROJ>
-__host__ __device__ constexpr int dense_bn() { return 4 * 16 * dense_rt<FMT, NPROJ>(); }
+__host__ __device__ constexpr int dense_bn() { return FMT::XSUM ? 128 : 64 * dense_mx_rt<NPROJ>(); }   // rows per block
 
-template <class FMT, int NPROJ, int NT>
+template <int NPROJ>
 __global__ void __launch_bounds__(256, 2) k_dense(TileArgs a) {
-    constexpr bool INT4 = FMT::XSUM;
-    constexpr int SPG = INT4 ? 2 : 1;     // MFMA steps (32 inputs) per scale group
-    constexpr int RT = dense_rt<FMT, NPROJ>();   // 16-row tiles per projection per wave
+    using FMT = FmtMxfp4;
+    constexpr int NT = 4;                 // token tiles per pass
+    constexpr int RT = dense_mx_rt<NPROJ>();
     constexpr int BM = 16 * NT;           // tokens per pass
-    constexpr int BN = dense_bn<FMT, NPROJ>();   // rows per block (per projection)
+    constexpr int BN = dense_bn<FMT, NPROJ>();
     constexpr int SB = tile_slice_bytes<FMT>();
-    // int4 (F16): activations travel as fp16 with power-of-two exponents (x16 per token; h16 per slot) and the
-    // codes are dequantised to fp16 in registers; MXFP4 keeps the exact raw-code path on bf16 MFMA with its
-    // per-group fold (its E8M0 scales do not fit fp16), h = hi + lo
-    constexpr bool F16 = INT4;
-    constexpr bool H16 = INT4;
-    constexpr int HL = (NPROJ == 2 || H16) ? 1 : 2;   // activation planes: x, x16, h16, or h = hi + lo
+    constexpr int HL = NPROJ == 2 ? 1 : 2;   // activation planes: x, or h = hi + lo
     constexpr int NDMA = BM / 16;         // DMA instructions per wave per slice and plane (4 token rows each)
     __shared__ __attribute__((aligned(1024))) uint8_t sX0[HL * BM * 256];
     __shared__ __attribute__((aligned(1024))) uint8_t sX1[HL * BM * 256];
     __shared__ int sSlot[BM];
 
-    // Work items (pass list x row blocks x K parts), ordered expert by expert, within an expert row block by row
-    // block with the expert's passes adjacent, K part fastest. The launch hands workgroups to the 8 XCDs round
-    // robin (workgroup b to XCD (b + c) mod 8, c fixed per launch), so XCD slot b & 7 takes the contiguous
-    // eighth of the live items, in order: each XCD's L2 then holds the activations of few experts, and the
-    // passes that share a weight tile run side by side on one XCD (their second reads hit its L2). The grid is
-    // a multiple of 8 covering the largest possible item count.
+    // work items and their order: as in k_dense_i4
     const int nrb = (a.N + BN - 1) / BN;
     const int nitems = a.meta[a.nidx] * nrb * a.ksplit;
     const int chunk = (nitems + 7) >> 3;
     const int rank = (int)(blockIdx.x >> 3);
     const int item = (int)(blockIdx.x & 7u) * chunk + rank;
     if (rank >= chunk || item >= nitems) return;
-    const int ks = item % a.ksplit;               // K part (down only), the fastest index
-    const int bid = item / a.ksplit;
+    const int ks = item % a.ksplit, bid = item / a.ksplit;   // K part (down only), the fastest index
     const int wq = bid / nrb;                      // some pass of the current expert
     const int e = a.items[3 * wq], np = a.items[3 * wq + 2];
     const int w0 = wq - a.items[3 * wq + 1];       // the expert's first pass
@@ -1077,336 +1052,145 @@ __global__ void __launch_bounds__(256, 2) k_dense(TileArgs a) {
     if (HL == 2) xb[HL - 1] = reinterpret_cast<const uint8_t*>(a.actv2);
     // the DMA lanes: instruction i of this wave writes token rows 4 (wave + 4 i) + (lane >> 4), position lane & 15
     const int psw = (lane & 15) ^ ((4 * wave + (lane >> 4)) & 15);   // piece loaded by this lane
-    const uint32_t ones = 0x3F803F80u;
-    const bf16x8 ONES = as_bf16x8(ones, ones, ones, ones);
-
-    {
-        const int ntiles = (nlive + 15) >> 4;
-        if (tid < BM) sSlot[tid] = a.sorted[beg + (tok0 + tid < n ? tok0 + tid : n - 1)];
-        __syncthreads();
-        uint32_t xrow[NDMA];
+    const int ntiles = (nlive + 15) >> 4;
+    if (tid < BM) sSlot[tid] = a.sorted[beg + (tok0 + tid < n ? tok0 + tid : n - 1)];
+    __syncthreads();
+    uint32_t xrow[NDMA];
 #pragma unroll
-        for (int i = 0; i < NDMA; ++i)
-            xrow[i] = (uint32_t)(sSlot[4 * (wave + 4 * i) + (lane >> 4)] / a.act_div) * (uint32_t)K * 2u;
-        auto dma = [&](int s, uint8_t* buf) __attribute__((always_inline)) {
-            int piece = 16 * s + psw;
-            piece = piece < lastp ? piece : lastp;   // inputs past K meet zero codes and zero metadata
+    for (int i = 0; i < NDMA; ++i)
+        xrow[i] = (uint32_t)(sSlot[4 * (wave + 4 * i) + (lane >> 4)] / a.act_div) * (uint32_t)K * 2u;
+    auto dma = [&](int s, uint8_t* buf) __attribute__((always_inline)) {
+        int piece = 16 * s + psw;
+        piece = piece < lastp ? piece : lastp;   // inputs past K meet zero codes and zero metadata
 #pragma unroll
-            for (int hl = 0; hl < HL; ++hl)
+        for (int hl = 0; hl < HL; ++hl)
 #pragma unroll
-                for (int i = 0; i < NDMA; ++i) {
-                    // 32-bit offset from the uniform base (kept opaque so no 64-bit address is held per row)
-                    uint32_t o = xrow[i];
-                    asm volatile("" : "+v"(o));
-                    __builtin_amdgcn_global_load_lds((const void*)(xb[hl] + (o + 16u * (uint32_t)piece)),
-                                                     MOE_LDSP(buf + (hl * BM + 4 * (wave + 4 * i)) * 256), 16, 0, 0);
-                }
-        };
-        uint4 rq[2][NPROJ][RT];
-        uint2 rm[2][NPROJ][RT];
-        // F16: entry h of lane j holds the exponent E of token 64 h + j of the pass: its activation row is x 2^-E
-        // (x16, k_x16) or h 2^-E (h16, k_h16_fix)
-        constexpr int NE = (BM + 63) / 64;   // lane j of entry h: token 64 h + j
-        int eslot[NE];
-#pragma unroll
-        for (int h = 0; h < NE; ++h) {
-            eslot[h] = 0;
-            const int j = 64 * h + lane;
-            if (F16 && j < BM) {
-                if (NPROJ == 1)
-                    eslot[h] = reinterpret_cast<const int32_t*>(reinterpret_cast<const uint8_t*>(a.actv2) + a.eslot_off)[sSlot[j]];
-                else
-                    eslot[h] = a.xexp[sSlot[j] / a.act_div];
+            for (int i = 0; i < NDMA; ++i) {
+                // 32-bit offset from the uniform base (kept opaque so no 64-bit address is held per row)
+                uint32_t o = xrow[i];
+                asm volatile("" : "+v"(o));
+                __builtin_amdgcn_global_load_lds((const void*)(xb[hl] + (o + 16u * (uint32_t)piece)),
+                                                 MOE_LDSP(buf + (hl * BM + 4 * (wave + 4 * i)) * 256), 16, 0, 0);
             }
-        }
-        auto wissue = [&](int s, uint4 (&q)[NPROJ][RT], uint2 (&m)[NPROJ][RT]) __attribute__((always_inline)) {
+    };
+    uint4 rq[2][NPROJ][RT];
+    uint32_t rm[2][NPROJ][RT];
+    auto wissue = [&](int s, uint4 (&q)[NPROJ][RT], uint32_t (&m)[NPROJ][RT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const uint8_t* sl = tb[p][rt] + (uint32_t)s * (uint32_t)SB;
+                q[p][rt] = *reinterpret_cast<const uint4*>(sl + 16 * lane);
+                m[p][rt] = *reinterpret_cast<const uint32_t*>(sl + 1024 + 4 * lr);
+            }
+    };
+    f32x4 acc[NPROJ][RT][NT];
+#pragma unroll
+    for (int p = 0; p < NPROJ; ++p)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[p][rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // one slice, scale group by scale group; lane (m, g) of MFMA step j supplies word 4 j + g of its row (the record
+    // order). FULL: every token tile of the pass is live (no branch inside the slice)
+    auto compute = [&](auto full, const uint8_t* xs, const uint4 (&q)[NPROJ][RT], const uint32_t (&m)[NPROJ][RT])
+                       __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            __builtin_amdgcn_sched_barrier(0);   // one group at a time: bounds the live operands
+            bf16x8 B[NPROJ][RT];
+            float ms[NPROJ][RT];
 #pragma unroll
             for (int p = 0; p < NPROJ; ++p)
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
-                    const uint8_t* sl = tb[p][rt] + (uint32_t)s * (uint32_t)SB;
-                    q[p][rt] = *reinterpret_cast<const uint4*>(sl + 16 * lane);
-                    if (INT4) m[p][rt] = *reinterpret_cast<const uint2*>(sl + 1024 + 8 * lr);
-                    else m[p][rt].x = *reinterpret_cast<const uint32_t*>(sl + 1024 + 4 * lr);
+                    const uint32_t w = j == 0 ? q[p][rt].x : (j == 1 ? q[p][rt].y : (j == 2 ? q[p][rt].z : q[p][rt].w));
+                    uint32_t c4[4];
+                    FMT::decode_word(w, c4);
+                    B[p][rt] = as_bf16x8(c4[0], c4[1], c4[2], c4[3]);
+                    ms[p][rt] = __uint_as_float(((m[p][rt] >> (8 * j)) & 0xFFu) << 23);
                 }
-        };
-        f32x4 acc[NPROJ][RT][NT];
 #pragma unroll
-        for (int p = 0; p < NPROJ; ++p)
+            for (int t = 0; t < NT; ++t) {
+                if (decltype(full)::value || t < ntiles) {   // wave-uniform
+                    bf16x8 A[HL];
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int t = 0; t < NT; ++t) acc[p][rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // F16 (int4): the B operands of projection p, row tile rt, scale group G, as fp16 w' = (s q + b) 2^-16 in
-        // one rounding: each code pair (q_k, q_{k+4}) is masked into bits 4-7 of two fp16 halves with exponent 0,
-        // which makes them the exact subnormals q 2^-20 (one shift and one mask), and one v_pk_fma_f16 takes
-        // q 2^-20 (16 s) + b 2^-16. The records' row scaling keeps |s|, |b| below 2^11, so 16 s < 2^15 fits fp16 and
-        // |w'| < 2^-1: a weight stays a normal fp16 number down to 2^-13 of that bound, and below it rounds to fp16's
-        // subnormal step 2^-24 (2^-19 of the row's largest |s|, |b| in w' units). The epilogue adds 16 to the row
-        // exponent. 11 VALU per code word. (Codes left in bits 0-3 as q 2^-24 save two shifts, 9 VALU, but bound
-        // |w'| by 2^-5 and so put weights 2^9 below the row's largest into the subnormal range: one group per row at
-        // 64x the others' scale and small x on it then reached 8e-3 of the output RMS in a numpy emulation, 4e-2 at
-        // 256x, against 5e-7 and 1.4e-3 for this decode.)
-        constexpr int DEC_EXP = 16;
-        auto decode_f16 = [&](int G, int p, int rt, const uint4 (&q)[NPROJ][RT], const uint2 (&m)[NPROJ][RT],
-                              f16x8 (&B)[NPROJ][RT][2]) __attribute__((always_inline)) {
-            const uint32_t mw = G ? m[p][rt].y : m[p][rt].x;
-            const _Float16 s16 = (_Float16)(bf16lo(mw) * 16.0f), b16 = (_Float16)(bf16hi(mw) * 0x1p-16f);
-            const h2x s2 = {s16, s16}, b2 = {b16, b16};
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int j = 2 * G + u;
-                const uint32_t w = j == 0 ? q[p][rt].x : (j == 1 ? q[p][rt].y : (j == 2 ? q[p][rt].z : q[p][rt].w));
-                const uint32_t c4[4] = {(w << 4) & 0x00F000F0u, w & 0x00F000F0u, (w >> 4) & 0x00F000F0u,
-                                        (w >> 8) & 0x00F000F0u};
-                h2x v[4];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) v[c] = __builtin_elementwise_fma(__builtin_bit_cast(h2x, c4[c]), s2, b2);
-                B[p][rt][u] = f16x8{v[0][0], v[0][1], v[1][0], v[1][1], v[2][0], v[2][1], v[3][0], v[3][1]};
-            }
-        };
-        // one slice as 2 NT steps f = G NT + t (scale group G, token tile t): group G's MFMAs (f16 x f16, fp32
-        // accumulate, straight into acc) for token tile t; after each of group 0's steps, group 1's (projection,
-        // row tile) pairs t * NPROJ * RT / NT ... are decoded, so that VALU work issues while MFMAs run. The A
-        // operands of step f + 2 are read from LDS while step f's MFMAs run, across the group boundary (three
-        // register sets; one step's MFMAs alone do not cover the LDS latency when a wave has only 2 row tiles), so
-        // a slice waits for LDS reads once, before its first step.
-        auto slice_f16 = [&](auto full, const uint8_t* xs, const uint4 (&q)[NPROJ][RT], const uint2 (&m)[NPROJ][RT])
-                             __attribute__((always_inline)) {
-            static_assert(NPROJ * RT % NT == 0 || NT % (NPROJ * RT) == 0, "decode pairs spread evenly over the token tiles");
-            // pairs decoded after each token tile (PPT >= 1), or one pair after every TPP-th token tile
-            constexpr int PPT = NPROJ * RT >= NT ? NPROJ * RT / NT : 1;
-            constexpr int TPP = NPROJ * RT >= NT ? 1 : NT / (NPROJ * RT);
-            constexpr int NS = 2 * NT;
-            f16x8 B0[NPROJ][RT][2], B1[NPROJ][RT][2];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int i = 0; i < NPROJ * RT; ++i) decode_f16(0, i / RT, i % RT, q, m, B0);
-            __builtin_amdgcn_sched_barrier(0);
-            auto live = [&](int f) __attribute__((always_inline)) { return decltype(full)::value || f % NT < ntiles; };
-            auto load_a = [&](int f, f16x8 (&A)[2]) __attribute__((always_inline)) {
-                const int G = f / NT, t = f % NT;
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    const int j = 2 * G + u;
-                    const int wi = j < 2 ? 2 * lg + j : 8 + 2 * lg + (j - 2);
-                    A[u] = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4*>(xs + (16 * t + lr) * 256 + 16 * (wi ^ lr)));
-                }
-            };
-            f16x8 Ab[3][2];
-            if (live(0)) load_a(0, Ab[0]);
-            if (live(1)) load_a(1, Ab[1]);
-#pragma unroll
-            for (int f = 0; f < NS; ++f) {
-                const int G = f / NT, t = f % NT;
-                if (f + 2 < NS && live(f + 2)) load_a(f + 2, Ab[(f + 2) % 3]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (live(f)) {   // wave-uniform
-#pragma unroll
-                    for (int u = 0; u < 2; ++u)
-#pragma unroll
-                        for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-                            for (int rt = 0; rt < RT; ++rt)
-                                acc[p][rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                    Ab[f % 3][u], G ? B1[p][rt][u] : B0[p][rt][u], acc[p][rt][t], 0, 0, 0);
-                }
-                if (G == 0 && t % TPP == TPP - 1) {
-#pragma unroll
-                    for (int i = (t / TPP) * PPT; i < (t / TPP + 1) * PPT; ++i) decode_f16(1, i / RT, i % RT, q, m, B1);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-        // one slice, scale group by scale group; lane (m, g) of MFMA step j supplies word wi(j, g) of its row
-        // (the record order). FULL: every token tile of the pass is live (no branch inside the slice)
-        auto compute = [&](auto full, const uint8_t* xs, const uint4 (&q)[NPROJ][RT], const uint2 (&m)[NPROJ][RT],
-                           int) __attribute__((always_inline)) {
-            if constexpr (F16) {
-                slice_f16(full, xs, q, m);
-                return;
-            }
-#pragma unroll
-            for (int G = 0; G < 4 / SPG; ++G) {
-                __builtin_amdgcn_sched_barrier(0);   // one group at a time: bounds the live operands
-                bf16x8 B[NPROJ][RT][SPG];
-                float ms[NPROJ][RT], mc[NPROJ][RT];
-#pragma unroll
-                for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-                        for (int u = 0; u < SPG; ++u) {
-                            const int j = SPG * G + u;
-                            const uint32_t w = j == 0 ? q[p][rt].x : (j == 1 ? q[p][rt].y : (j == 2 ? q[p][rt].z : q[p][rt].w));
-                            uint32_t c4[4];
-                            FMT::decode_word(w, c4);
-                            B[p][rt][u] = as_bf16x8(c4[0], c4[1], c4[2], c4[3]);
-                        }
-                        if (INT4) {
-                            const uint32_t mw = G ? m[p][rt].y : m[p][rt].x;
-                            ms[p][rt] = bf16lo(mw);
-                            mc[p][rt] = __builtin_fmaf(-128.f, ms[p][rt], bf16hi(mw));
-                        } else {
-                            ms[p][rt] = __uint_as_float(((m[p][rt].x >> (8 * G)) & 0xFFu) << 23);
-                            mc[p][rt] = 0.f;
-                        }
+                    for (int hl = 0; hl < HL; ++hl) {
+                        const uint4 av = *reinterpret_cast<const uint4*>(xs + (hl * BM + 16 * t + lr) * 256 +
+                                                                         16 * ((4 * j + lg) ^ lr));
+                        A[hl] = as_bf16x8(av.x, av.y, av.z, av.w);
                     }
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    if (decltype(full)::value || t < ntiles) {   // wave-uniform
-                        bf16x8 A[HL][SPG];
+                    for (int p = 0; p < NPROJ; ++p)
 #pragma unroll
-                        for (int hl = 0; hl < HL; ++hl)
-#pragma unroll
-                            for (int u = 0; u < SPG; ++u) {
-                                const int j = SPG * G + u;
-                                const int wi = INT4 ? (j < 2 ? 2 * lg + j : 8 + 2 * lg + (j - 2)) : 4 * j + lg;
-                                const uint4 av = *reinterpret_cast<const uint4*>(
-                                    xs + (hl * BM + 16 * t + lr) * 256 + 16 * (wi ^ lr));
-                                A[hl][u] = as_bf16x8(av.x, av.y, av.z, av.w);
-                            }
-                        f32x4 xsum = f32x4{0.f, 0.f, 0.f, 0.f};
-                        if (INT4) {
+                        for (int rt = 0; rt < RT; ++rt) {
+                            f32x4 P = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                             for (int hl = 0; hl < HL; ++hl)
+                                P = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[hl], B[p][rt], P, 0, 0, 0);
 #pragma unroll
-                                for (int u = 0; u < SPG; ++u)
-                                    xsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[hl][u], ONES, xsum, 0, 0, 0);
+                            for (int v = 0; v < 4; ++v)
+                                acc[p][rt][t][v] = __builtin_fmaf(ms[p][rt], P[v], acc[p][rt][t][v]);
                         }
-#pragma unroll
-                        for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-                            for (int rt = 0; rt < RT; ++rt) {
-                                f32x4 P = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                                for (int hl = 0; hl < HL; ++hl)
-#pragma unroll
-                                    for (int u = 0; u < SPG; ++u)
-                                        P = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[hl][u], B[p][rt][u], P, 0, 0, 0);
-#pragma unroll
-                                for (int v = 0; v < 4; ++v) {
-                                    if (INT4)
-                                        acc[p][rt][t][v] = __builtin_fmaf(ms[p][rt], P[v],
-                                                                          __builtin_fmaf(mc[p][rt], xsum[v], acc[p][rt][t][v]));
-                                    else
-                                        acc[p][rt][t][v] = __builtin_fmaf(ms[p][rt], P[v], acc[p][rt][t][v]);
-                                }
-                            }
-                    }
                 }
             }
-        };
-        // int4: row exponents of the lane's rows (the records hold s 2^-E, b 2^-E; the epilogue scales by 2^E)
-        int rex[NPROJ][RT];
-#pragma unroll
-        for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-                rex[p][rt] = INT4 && wvalid ? tile_row_exps(p ? a.W1 : a.W0, a.E, N, K)[(size_t)e * N + r0 + 16 * rt + lr] + DEC_EXP : 0;
-        // slice s sits in buffer / ring slot s & 1; slice s + 1 is fetched during slice s (the last slice fetches
-        // itself again into the idle slot: no branch around the loads)
-        auto run = [&](auto full) __attribute__((always_inline)) {
-            dma(sb0, sX0);
-            wissue(sb0, rq[0], rm[0]);
+        }
+    };
+    // slice s sits in buffer / ring slot s & 1; slice s + 1 is fetched during slice s (the last slice fetches
+    // itself again into the idle slot: no branch around the loads)
+    auto run = [&](auto full) __attribute__((always_inline)) {
+        dma(sb0, sX0);
+        wissue(sb0, rq[0], rm[0]);
+        MOE_VMWAIT0();
+        MOE_BARRIER();
+        int j = 0;
+        for (; j + 2 <= scnt; j += 2) {
+            wissue(sb0 + j + 1, rq[1], rm[1]);
+            dma(sb0 + j + 1, sX1);
+            compute(full, sX0, rq[0], rm[0]);
             MOE_VMWAIT0();
             MOE_BARRIER();
-            int j = 0;
-            for (; j + 2 <= scnt; j += 2) {
-                wissue(sb0 + j + 1, rq[1], rm[1]);
-                dma(sb0 + j + 1, sX1);
-                compute(full, sX0, rq[0], rm[0], j);
-                MOE_VMWAIT0();
-                MOE_BARRIER();
-                const int jn = sb0 + (j + 2 < scnt ? j + 2 : j + 1);
-                wissue(jn, rq[0], rm[0]);
-                dma(jn, sX0);
-                compute(full, sX1, rq[1], rm[1], j + 1);
-                MOE_VMWAIT0();
-                MOE_BARRIER();
-            }
-            if (j < scnt) compute(full, sX0, rq[0], rm[0], j);   // odd count: the last slice is in slot 0
-        };
-        if (ntiles == NT) run(std::true_type{});
-        else run(std::false_type{});
-
-        // ---- epilogue: lane holds row r0 + 16 rt + lr of tokens tok0 + 16 t + 4 lg + v
-        if constexpr (H16 && NPROJ == 2) {
-            // h of the wave's 32 rows as fp16 h16 = h 2^-e, e per token: 0 while |h| < 2^15 on those rows, else
-            // the power of two that brings their largest |h| below 2^15 (so fp16 never overflows); e goes to the
-            // exponent bytes [slot, F / 32] (one 32-row chunk per wave)
-            static_assert(RT == 2, "one 32-row chunk per wave");
-            float hv[NT][4][RT];
-            int xe[NT][4];   // x16 = x 2^-E per token: the sums are scaled back before the GLU
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) xe[t][v] = __shfl(eslot[(16 * t) >> 6], (16 * t + 4 * lg + v) & 63, 64);
-            int8_t* hexp_out = reinterpret_cast<int8_t*>(a.hout2);
-            const int nch = N >> 5;
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    float am = 0.f;
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) {
-                        const int r = r0 + 16 * rt + lr;
-                        float g = __builtin_ldexpf(acc[0][rt][t][v], xe[t][v] + rex[0][rt]);
-                        float up = __builtin_ldexpf(acc[1][rt][t][v], xe[t][v] + rex[1][rt]);
-                        if (wvalid && a.b0) g += a.b0[(size_t)e * N + r];
-                        if (wvalid && a.b1) up += a.b1[(size_t)e * N + r];
-                        hv[t][v][rt] = wvalid ? glu_act(a.act, g, up) : 0.f;
-                        am = fmaxf(am, fabsf(hv[t][v][rt]));
-                    }
-#pragma unroll
-                    for (int o = 1; o < 16; o <<= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
-                    const int ex = h16_exponent(am);
-                    const int jt = 16 * t + 4 * lg + v;
-                    if (jt >= nlive || !wvalid) continue;
-                    const int slot = sSlot[jt];
-                    if (lr == 0) hexp_out[(size_t)slot * nch + (r0 >> 5)] = (int8_t)ex;
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) {
-                        const _Float16 h16 = (_Float16)__builtin_ldexpf(hv[t][v][rt], -ex);
-                        a.hout[(size_t)slot * N + r0 + 16 * rt + lr] = __builtin_bit_cast(uint16_t, h16);
-                    }
-                }
-        } else {
-            int es[NT][4];   // H16 down: the exponent of each of the lane's tokens (all lanes take part in the shuffle)
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) es[t][v] = H16 ? __shfl(eslot[(16 * t) >> 6], (16 * t + 4 * lg + v) & 63, 64) : 0;
-            if (wvalid)
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int jt = 16 * t + 4 * lg + v;
-                    if (jt >= nlive) continue;
-                    const int slot = sSlot[jt];
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt) {
-                        const int r = r0 + 16 * rt + lr;
-                        if (NPROJ == 2) {
-                            float g = acc[0][rt][t][v], up = acc[NPROJ - 1][rt][t][v];
-                            if (a.b0) g += a.b0[(size_t)e * N + r];
-                            if (a.b1) up += a.b1[(size_t)e * N + r];
-                            const float hv = glu_act(a.act, g, up);
-                            const uint16_t hi = f32_to_bf16(hv);
-                            a.hout[(size_t)slot * N + r] = hi;
-                            a.hout2[(size_t)slot * N + r] = f32_to_bf16(hv - bf16_to_f32(hi));
-                        } else if (H16) {
-                            a.yp[ks * a.plane + (size_t)slot * N + r] = __builtin_ldexpf(acc[0][rt][t][v], es[t][v] + rex[0][rt]);
-                        } else {
-                            a.yp[ks * a.plane + (size_t)slot * N + r] = acc[0][rt][t][v];
-                        }
-                    }
-                }
+            const int jn = sb0 + (j + 2 < scnt ? j + 2 : j + 1);
+            wissue(jn, rq[0], rm[0]);
+            dma(jn, sX0);
+            compute(full, sX1, rq[1], rm[1]);
+            MOE_VMWAIT0();
+            MOE_BARRIER();
         }
-    }
+        if (j < scnt) compute(full, sX0, rq[0], rm[0]);   // odd count: the last slice is in slot 0
+    };
+    if (ntiles == NT) run(std::true_type{});
+    else run(std::false_type{});
+
+    // ---- epilogue: lane holds row r0 + 16 rt + lr of tokens tok0 + 16 t + 4 lg + v
+    if (!wvalid) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int jt = 16 * t + 4 * lg + v;
+            if (jt >= nlive) continue;
+            const int slot = sSlot[jt];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const int r = r0 + 16 * rt + lr;
+                if (NPROJ == 2) {
+                    float g = acc[0][rt][t][v], up = acc[NPROJ - 1][rt][t][v];
+                    if (a.b0) g += a.b0[(size_t)e * N + r];
+                    if (a.b1) up += a.b1[(size_t)e * N + r];
+                    const float hv = glu_act(a.act, g, up);
+                    const uint16_t hi = f32_to_bf16(hv);
+                    a.hout[(size_t)slot * N + r] = hi;
+                    a.hout2[(size_t)slot * N + r] = f32_to_bf16(hv - bf16_to_f32(hi));
+                } else {
+                    a.yp[ks * a.plane + (size_t)slot * N + r] = acc[0][rt][t][v];
+                }
+            }
+        }
 }
+
+#include "moe_dense_i4.h"
 
 // ============================================================================ MXFP4 dense tiles on the block-scaled MFMA
 // gfx950's v_mfma_scale_f32_16x16x128_f8f6f4 multiplies fp8 (E4M3) A by fp4 (E2M1) B over 128 inputs, each
@@ -1972,18 +1756,27 @@ int dense_ksplit(int N, int K, int nslots, int E, int BN, int P) {
     return (nsl + per - 1) / per;
 }
 
-template <class FMT, int NPROJ, int NT = dense_nt<FMT, NPROJ>()>
+template <int NPROJ>
 int launch_dense(TileArgs t, int nslots, hipStream_t st) {
-    constexpr int BN = dense_bn<FMT, NPROJ>();
-    if (t.N % (16 * dense_rt<FMT, NPROJ>())) return MOE_ERR_ARG;   // whole row tiles per wave
-    if (NPROJ == 2) t.ksplit = 1;
+    constexpr int BN = dense_bn<FmtMxfp4, NPROJ>();
+    if (t.N % (16 * dense_mx_rt<NPROJ>())) return MOE_ERR_ARG;   // whole row tiles per wave
     // rounded up to a multiple of 8: every XCD slot then has a workgroup for each of its ceil(items / 8) items
-    const long nblk = ((long)((t.N + BN - 1) / BN) * max_passes(nslots, t.E, 16 * NT) * t.ksplit + 7) / 8 * 8;
+    if (NPROJ == 2) t.ksplit = 1;
+    const long nblk = ((long)((t.N + BN - 1) / BN) * max_passes(nslots, t.E, 64) * t.ksplit + 7) / 8 * 8;
     if (nblk > 0x7FFFFFF8L) return MOE_ERR_ARG;
-    k_dense<FMT, NPROJ, NT><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
+    k_dense<NPROJ><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
-
+template <int NPROJ, int RT, int M, int MINB>
+int launch_dense_i4(TileArgs t, int nslots, hipStream_t st) {
+    constexpr int BN = 128 * RT;
+    if (t.N % (32 * RT)) return MOE_ERR_ARG;   // whole row tiles per wave
+    if (NPROJ == 2) t.ksplit = 1;
+    const long nblk = ((long)((t.N + BN - 1) / BN) * max_passes(nslots, t.E, 64) * t.ksplit + 7) / 8 * 8;
+    if (nblk > 0x7FFFFFF8L) return MOE_ERR_ARG;
+    k_dense_i4<NPROJ, RT, M, MINB><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
+    return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
+}
 
 #ifndef MOE_DENSE_MIN_BLOCKS
 #define MOE_DENSE_MIN_BLOCKS 256   // dense gate/up blocks below which the wave tiles fill the chip better
@@ -1998,7 +1791,7 @@ int launch_dense(TileArgs t, int nslots, hipStream_t st) {
 // down, on two pass lists.
 struct Plan {
     bool tiled, dense_gu, dense_dn, mxd, wave_gu, wave_dn, mxw, h16, two_lists, ingroup;
-    int nt, dn_nt, P_gu, P_dn;
+    int nt, i4_m, P_gu, P_dn;
 };
 
 template <class FMT>
@@ -2010,10 +1803,10 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
     constexpr bool INT4 = FmtInt4::FMT == FMT::FMT;
     p.tiled = w->gate.tiles && w->up.tiles && w->down.tiles;
     const int dmode = env_int("MOE_DENSE", -1);
-    constexpr int DP_GU = 16 * dense_nt<FMT, 2>(), DP_DN = 16 * dense_nt<FMT, 1>();
+    constexpr int DP = 64;   // the dense tiles' pass
     constexpr int BN_GU = dense_bn<FMT, 2>(), BN_DN = dense_bn<FMT, 1>();
-    const long dblocks = (long)((w->F + BN_GU - 1) / BN_GU) * max_passes(nslots, w->E, DP_GU);
-    const long dn_blocks = (long)((w->d + BN_DN - 1) / BN_DN) * max_passes(nslots, w->E, DP_DN);
+    const long dblocks = (long)((w->F + BN_GU - 1) / BN_GU) * max_passes(nslots, w->E, DP);
+    const long dn_blocks = (long)((w->d + BN_DN - 1) / BN_DN) * max_passes(nslots, w->E, DP);
     const int min_avg = env_int("MOE_DENSE_MIN_AVG", 32);
     const int dn_min_avg = env_int("MOE_DENSE_DN_MIN_AVG", 16);
     // activations as planes (fp16 / fp32 x): the dense gate/up takes only what it reads exactly, int4 with fp16 x
@@ -2041,17 +1834,16 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
     p.nt = nx > 1 ? 1
          : (p.wave_gu || p.wave_dn) ? (wnt == 1 || wnt == 2 ? wnt : (avg <= 16 ? 1 : 2))
                                     : tokens_per_pass_tiles(T, k, w->E);
-    // pass lists: 16 nt tokens per pass for the wave tiles, DP_GU / 16 dn_nt for the dense tiles; a second list
-    // when the two stages take different kernels
-    // the int4 dense down's pass: 64 tokens (MOE_DENSE_DN_NT = 2, 4, 8 token tiles for A/B runs). Against 128-token
-    // passes (each decoded weight tile feeding 8 token tiles, 64 accumulators, 2 waves per SIMD) the 64-token pass
-    // runs 4 waves per SIMD (128 VGPRs) and, with twice the items, no K split: DeepSeek-V2-Lite T=256 (31 slots per
-    // expert, where a 128-token pass decodes its tiles for 2 live token tiles) 166-168 -> 148-149 us per layer,
-    // Mixtral T=512 655-672 -> 638-650 us (32-token passes: 147-153 and 682-696 us)
-    const int dnt = env_int("MOE_DENSE_DN_NT", 0);
-    p.dn_nt = !INT4 ? dense_nt<FMT, 1>() : (dnt == 2 || dnt == 4 || dnt == 8) ? dnt : 4;
-    p.P_gu = p.dense_gu ? DP_GU : 16 * p.nt;
-    p.P_dn = p.dense_dn ? 16 * p.dn_nt : 16 * p.nt;
+    // the int4 dense gate/up's token tile: 16 tokens up to 48 slots per expert on average (three quarters of a 64-token
+    // pass: tiles of 32 would be a third empty), else 32 (fewer registers: three blocks per CU). Layer times, 16 / 32:
+    // OLMoE T = 272 (34 slots) 97.2 / 99.8 us, T = 333 (42) 94.9 / 101.7, Mixtral T = 160 (40) 227 / 248; OLMoE T = 512
+    // (64) 140 / 132, Qwen3 T = 544 (34, skew apart) 148.6 / 146.0, d = 1088 F = 704 T = 700 (53) 66.9 / 55.9, Mixtral
+    // T = 512 (128) 486 / 484
+    p.i4_m = avg <= 48 ? 16 : 32;
+    // pass lists: 16 nt tokens per pass for the wave tiles, 64 for the dense tiles; a second list when the two stages
+    // take different kernels
+    p.P_gu = p.dense_gu ? DP : 16 * p.nt;
+    p.P_dn = p.dense_dn ? DP : 16 * p.nt;
     p.two_lists = p.P_gu != p.P_dn;
     // both stages on the wave tiles with few slots: each workgroup can find its pass from the raw ids itself (an LDS
     // histogram and a wave scan, the grouping launch's order), so the call needs no grouping launch
@@ -2149,7 +1941,11 @@ int run_tiles_fmt(const ExpertsArgs& a) {
             g.actv = reinterpret_cast<const uint16_t*>(a.xterm);
             if (!rc) rc = launch_wave_tile<FMT, 2, MOE_WAVE_RT_GU, MOE_WAVE_D_GU>(g, nt, nslots, a.st, 1, 2);
         } else if (mxd) rc = 0;
-        else if (dense_gu) rc = launch_dense<FMT, 2>(g, nslots, a.st);
+        else if (dense_gu) {
+            if constexpr (!INT4) rc = launch_dense<2>(g, nslots, a.st);
+            else if (pl.i4_m == 16) rc = launch_dense_i4<2, 1, 16, 2>(g, nslots, a.st);
+            else rc = launch_dense_i4<2, 1, 32, 3>(g, nslots, a.st);
+        }
         else if (wave_gu && h16)
             rc = launch_wave_tile<FMT, 2, MOE_WAVE_RT_GU, MOE_WAVE_D_GU, INT4>(g, nt, nslots, a.st, a.nx);
         else if (wave_gu) rc = launch_wave_tile<FMT, 2, MOE_WAVE_RT_GU, MOE_WAVE_D_GU>(g, nt, nslots, a.st, a.nx);
@@ -2193,13 +1989,10 @@ int run_tiles_fmt(const ExpertsArgs& a) {
             d.W0 = (const uint8_t*)w->down.tiles;
             rc = launch_mxd<1, 3>(d, nslots, a.st);
         } else if (dense_dn) {
-            if constexpr (INT4) {
-                if (pl.dn_nt == 2) rc = launch_dense<FMT, 1, 2>(d, nslots, a.st);
-                else if (pl.dn_nt == 4) rc = launch_dense<FMT, 1, 4>(d, nslots, a.st);
-                else rc = launch_dense<FMT, 1>(d, nslots, a.st);
-            } else {
-                rc = launch_dense<FMT, 1>(d, nslots, a.st);
-            }
+            // int4: 32 rows per wave at four blocks per CU; 64 rows (three blocks) or 32-token tiles measured slower on
+            // every shape but Qwen3 T = 4096 (even)
+            if constexpr (INT4) rc = launch_dense_i4<1, 1, 16, 4>(d, nslots, a.st);
+            else rc = launch_dense<1>(d, nslots, a.st);
         }
         else if (wave_dn && wide_dn(MOE_WAVE_RT_DN_WIDE))
             rc = launch_wave_tile<FMT, 1, MOE_WAVE_RT_DN_WIDE, MOE_WAVE_D_DN>(d, nt, nslots, a.st, 1, mxt);

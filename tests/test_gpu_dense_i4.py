@@ -1,0 +1,56 @@
+"""int4 dense tiles at the edges of their token tiles: counts per expert around multiples of 16, 32 and 64 (both token-tile
+sizes, one and several passes), ragged last row blocks, inputs that end at half a slice, one to many K slices, every GLU,
+fp16 and bf16 activations, against the CPU oracle at the dense tiles' gate."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_close, oracle_y
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _run(d, F, counts, act, dtype, seed):
+    """Experts with the given slot counts (k = 1), in shuffled token order."""
+    from moelab_amd import _lib, experts
+    from moelab_amd.problem import baseline_int4_layer
+    from moelab_amd.shapes import MoEShape
+    E, T = len(counts), sum(counts)
+    s = baseline_int4_layer(MoEShape("t", d=d, f=F, E=E, k=1), seed=seed, device=DEV, router=False)
+    rng = np.random.default_rng(seed)
+    idx = torch.from_numpy(rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts))[:, None].copy()).to(DEV)
+    wts = torch.from_numpy(rng.random((T, 1), dtype=np.float32)).to(DEV)
+    x = torch.from_numpy(rng.standard_normal((T, d), dtype=np.float32)).to(DEV).to(dtype)
+    print(f"case dense i4 d={d} F={F} counts={counts} act={act} {dtype}", flush=True)
+    y = experts.run_experts(s, x, idx, wts, act=act, path=_lib.PATH_GROUPED, out_dtype=torch.float32)
+    # fp16 weights and activations: 2^-12 per operand, a few thousand terms: well inside 5e-3 of the RMS
+    assert_close(y, oracle_y(s, x, idx, wts, act=act), tol=5e-3, what=(d, F, counts, act))
+
+
+@pytest.mark.parametrize("counts", [[47, 33, 48, 32, 1, 64, 65, 49], [31, 16, 17, 63, 15, 80, 81, 60],        # avg <= 48
+                                    [128, 129, 127, 64, 65, 33, 96, 1], [200, 1, 0, 191, 193, 63, 0, 97]])   # avg > 48
+@pytest.mark.parametrize("d,F,act,dtype", [(192, 320, 0, torch.bfloat16), (128, 64, 1, torch.float16),
+                                           (1088, 192, 2, torch.bfloat16)])
+def test_token_tile_edges(monkeypatch, counts, d, F, act, dtype):
+    monkeypatch.setenv("MOE_DENSE", "1")
+    _run(d, F, counts, act, dtype, seed=sum(counts) + d)
+
+
+def test_dead_tokens_and_large_h_write_only_their_slots(monkeypatch):
+    """h beyond fp16 (per-chunk exponents, the epilogue's scaled branch) beside ordinary tokens in one pass."""
+    from moelab_amd import _lib, experts
+    from moelab_amd.problem import baseline_int4_layer
+    from moelab_amd.shapes import MoEShape
+    monkeypatch.setenv("MOE_DENSE", "1")
+    d, F, E, T = 256, 192, 2, 150
+    s = baseline_int4_layer(MoEShape("t", d=d, f=F, E=E, k=1), seed=9, device=DEV, router=False)
+    x = torch.randn((T, d), device=DEV).to(torch.bfloat16)
+    x[::7] *= 3e3      # |h| to ~1e8
+    x[3::7] *= 1e-3    # chunks below 2^-8
+    idx = (torch.arange(T, device=DEV, dtype=torch.int32) % 3 == 0).to(torch.int32)[:, None].contiguous()
+    wts = torch.ones((T, 1), device=DEV)
+    y = experts.run_experts(s, x, idx, wts, path=_lib.PATH_GROUPED, out_dtype=torch.float32)
+    want = oracle_y(s, x, idx, wts)
+    for rows in (slice(0, None, 7), slice(3, None, 7), slice(1, None, 7)):
+        assert_close(y[rows], want[rows], tol=1e-2, what=rows)
