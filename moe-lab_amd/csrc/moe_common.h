@@ -84,6 +84,12 @@ __device__ __forceinline__ void load_x32(const uint16_t* p, uint32_t xw[16]) {
     }
 }
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);   // raw, bounds-checked
+}
+
 // ------------------------------------------------------------------------------------ DPP reductions
 // v + (v moved across lanes by a DPP pattern); lanes the pattern does not write add 0.
 template <int CTRL, int ROW_MASK = 0xF>
@@ -167,6 +173,19 @@ __device__ __forceinline__ uint32_t wave_umax_dpp(uint32_t v) {
     v = dpp_umax<0x143, 0xC>(v);
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
+// max over aligned groups of G = 16 or 32 lanes (v >= 0), in every lane: DPP within rows of 16, then pairs of rows
+template <int G>
+__device__ __forceinline__ float max_lanes(float v) {
+    v = dpp_max<0xB1>(v);
+    v = dpp_max<0x4E>(v);
+    v = dpp_max<0x141>(v);
+    v = dpp_max<0x140>(v);
+    if constexpr (G == 32) {
+        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
+    }
+    return v;
+}
 __device__ __forceinline__ float wave_sum_dpp(float v) {
     v = sum_lanes<64>(v);
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
@@ -238,6 +257,25 @@ __device__ __forceinline__ float glu(float g, float u) {
 
 __device__ __forceinline__ float glu_act(int act, float g, float u) {
     return act == 0 ? glu<0>(g, u) : (act == 1 ? glu<1>(g, u) : glu<2>(g, u));
+}
+
+// GLU on the transcendental unit's exp2 and reciprocal (about 1 ulp each, 1e-6 relative for large |g|), far below the
+// rounding of the h they feed (fp16, or three fp8 terms); sigmoid(x) from exp(-|x|), so nothing overflows. tanh-GELU through
+// (1 + tanh z) / 2 = sigmoid(2 z). With the libm forms the epilogue took as long as a third of a K = 2048 block's
+// products (Qwen3 T = 4096 gate/up 314 -> 280 us at 128-token passes).
+__device__ __forceinline__ float sigmoid_fast(float x) {
+    const float t = __builtin_amdgcn_exp2f(fabsf(x) * -1.44269504088896341f), r = __builtin_amdgcn_rcpf(1.f + t);
+    return x >= 0.f ? r : t * r;
+}
+__device__ __forceinline__ float glu_fast(int act, float g, float u) {
+    float z = g;
+    if (act == 1) z = 1.5957691216057308f * (g + 0.044715f * g * g * g);
+    if (act == 2) {
+        g = fminf(g, 7.f);
+        u = fminf(fmaxf(u, -7.f), 7.f) + 1.f;
+        z = 1.702f * g;
+    }
+    return g * sigmoid_fast(z) * u;
 }
 
 // ------------------------------------------------------------------------------------ GEMV pieces (T = 1 kernels)

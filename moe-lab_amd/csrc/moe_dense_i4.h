@@ -1,47 +1,6 @@
 // int4 dense tiles on fp16 MFMA (included by moe_tiles.hip after TileArgs): calls with many tokens per expert.
 #pragma once
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);   // raw, bounds-checked
-}
-
-// max over aligned groups of G = 16 or 32 lanes (v >= 0), in every lane: DPP within rows of 16, then pairs of rows
-template <int G>
-__device__ __forceinline__ float max_lanes(float v) {
-    v = dpp_max<0xB1>(v);
-    v = dpp_max<0x4E>(v);
-    v = dpp_max<0x141>(v);
-    v = dpp_max<0x140>(v);
-    if constexpr (G == 32) {
-        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
-    }
-    return v;
-}
-
-// GLU on the transcendental unit's exp2 and reciprocal (about 1 ulp each, 1e-6 relative for large |g|), far below the
-// fp16 rounding of the h16 they feed; sigmoid(x) from exp(-|x|), so nothing overflows. tanh-GELU through
-// (1 + tanh z) / 2 = sigmoid(2 z). With the libm forms the epilogue took as long as a third of a K = 2048 block's
-// products (Qwen3 T = 4096 gate/up 314 -> 280 us at 128-token passes).
-__device__ __forceinline__ float sigmoid_fast(float x) {
-    const float t = __builtin_amdgcn_exp2f(fabsf(x) * -1.44269504088896341f), r = __builtin_amdgcn_rcpf(1.f + t);
-    return x >= 0.f ? r : t * r;
-}
-__device__ __forceinline__ float glu_fast(int act, float g, float u) {
-    float z = g;
-    if (act == 1) z = 1.5957691216057308f * (g + 0.044715f * g * g * g);
-    if (act == 2) {
-        g = fminf(g, 7.f);
-        u = fminf(fmaxf(u, -7.f), 7.f) + 1.f;
-        z = 1.702f * g;
-    }
-    return g * sigmoid_fast(z) * u;
-}
-
 // A 4-wave block owns 128 RT rows of one expert (per projection) and one pass of up to 64 of its tokens, NT tiles of M;
 // wave w takes 32 RT of the rows for all the pass's tokens, so each weight is decoded once per pass. Per 128-input slice
 // the tokens' activations (x16 / h16, fp16) come into LDS by DMA and the wave's weight records into registers, both one

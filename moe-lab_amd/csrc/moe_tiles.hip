@@ -57,6 +57,7 @@ __device__ __forceinline__ int h16_exponent(float amax) {
     return 0;
 }
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int TL_ROWS = 64;   // weight rows per block
 constexpr int TL_KC = 8;      // chunks (32 inputs) per K slice
 constexpr int TL_APAD = 4 * TL_KC + 4;   // words per staged row: [g 0..3][chunk 0..KC-1] + 4 words of padding
@@ -64,45 +65,60 @@ constexpr int TL_BPAD = 4 * TL_KC + 1;   // 16-byte pieces per staged token (8 i
 constexpr int TL_GMAX = TL_KC;           // scale groups per slice at most (MXFP4: one per chunk)
 
 
-// Byte of record-term position of input k (0..127) of a slice: the code order of the tile records within each
-// word (inputs 8 i + (0 2 4 6 1 3 5 7)), then the A operand's lane order (bytes 32 g .. 32 g + 15: logical inputs
-// 16 g .. 16 g + 15, bytes 32 g + 16 .. 32 g + 31: 64 + 16 g .. 64 + 16 g + 15)
-__device__ __forceinline__ int mx_pos(int k) {
-    const int e = k & 7;
-    const int l = (k & ~7) | ((e >> 1) + 4 * (e & 1));
-    return 32 * ((l & 63) >> 4) + 16 * (l >> 6) + (l & 15);
-}
-
-// One token's h on the 32 rows of a wave's block b of slice s (lane lr of its lane group: rows 16 rt + lr of
-// the block, values h0 (rt 0) and h1 (rt 1)) -> the NTERM term bytes and scale bytes of that block in the token's
-// record rec (the layout k_mx_terms writes). The 16 lanes of the group take part in the max reductions; only
-// `write` lanes store. pad: also the zero blocks 2, 3 of a slice that ends at input 64 (K % 128 == 64).
-template <int NTERM>
-__device__ __forceinline__ void mx_h_block(float h0, float h1, bool write, uint8_t* rec, int b, int lr, bool pad) {
-    const int p0 = mx_pos(32 * b + lr), p1 = mx_pos(32 * b + 16 + lr);
+// h of a 16-token tile on the 32 rows of a wave's block b of slice s, as 3-term records (the layout k_mx_terms writes),
+// through LDS: mx_h_terms leaves each token's term bytes in a 112-byte LDS record (per term 32 bytes in the record's order,
+// then the three scale bytes), one byte per lane and row; mx_h_store copies them out 16 bytes per lane. Written from the
+// lanes directly they were byte stores, two per term and token.
+constexpr int MXH_REC = 112;
+// Lane lr of a lane group: rows 16 rt + lr of the block, values h0 (rt 0) and h1 (rt 1); the 16 lanes of the group take
+// part in the max reductions. rows 16 rt + lr sit at byte 16 rt + (lr & 8) + (0 4 1 5 2 6 3 7)[lr & 7] of a term's 32.
+__device__ __forceinline__ void mx_h_terms(float h0, float h1, uint8_t* ls, int lr) {
+    const int pos = (lr & 8) | (((lr & 7) >> 1) + 4 * (lr & 1));
 #pragma unroll
-    for (int t = 0; t < NTERM; ++t) {
-        float am = fmaxf(fabsf(h0), fabsf(h1));
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
+    for (int t = 0; t < 3; ++t) {
+        const float am = max_lanes<16>(fmaxf(fabsf(h0), fabsf(h1)));
         int e = am > 0.f ? (int)((__float_as_uint(am) >> 23) & 0xFFu) - 127 - 7 : -127;
         e = e < -127 ? -127 : (e > 127 ? 127 : e);
         const float inv = __builtin_ldexpf(1.f, -e);
         const uint32_t w = __builtin_amdgcn_cvt_pk_fp8_f32(h0 * inv, h1 * inv, 0, false);
         h0 -= __builtin_ldexpf(__builtin_amdgcn_cvt_f32_fp8((int)w, 0), e);
         h1 -= __builtin_ldexpf(__builtin_amdgcn_cvt_f32_fp8((int)w, 1), e);
-        if (write) {
-            rec[128 * t + p0] = (uint8_t)(w & 0xFFu);
-            rec[128 * t + p1] = (uint8_t)((w >> 8) & 0xFFu);
-            if (lr == 0) rec[128 * NTERM + 4 * t + b] = (uint8_t)(e + 127);
-        }
+        ls[32 * t + pos] = (uint8_t)(w & 0xFFu);
+        ls[32 * t + 16 + pos] = (uint8_t)((w >> 8) & 0xFFu);
+        if (lr == 0) ls[96 + t] = (uint8_t)(e + 127);
     }
-    if (pad && write && lr < 2 * NTERM) {   // blocks 2 and 3: lane lr zeroes term lr >> 1's block 2 + (lr & 1)
-        const int t = lr >> 1, bz = 2 + (lr & 1);
-        uint8_t* z = rec + 128 * t + 64 * (bz & 1) + 16 * (bz >> 1);
-        *reinterpret_cast<uint4*>(z) = uint4{0u, 0u, 0u, 0u};
-        *reinterpret_cast<uint4*>(z + 32) = uint4{0u, 0u, 0u, 0u};
-        rec[128 * NTERM + 4 * t + bz] = 127;
+}
+// One wave: tokens 0 .. nlive - 1 of the tile (slots slot_of(token), called by all lanes) to their records in hterm. pad:
+// also the zero blocks 2, 3 of a slice that ends at input 64 (K % 128 == 64).
+template <typename F>
+__device__ __forceinline__ void mx_h_store(const uint8_t* ls, int nlive, F slot_of, uint8_t* hterm, int nsl, int s, int b,
+                                           bool pad) {
+    constexpr int REC = mx_rec<3>();
+    const int lane = threadIdx.x & 63;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the lanes read one another's bytes
+    auto rec_of = [&](int tok) { return hterm + ((size_t)slot_of(tok) * nsl + s) * REC; };
+#pragma unroll
+    for (int i0 = 0; i0 < 128; i0 += 64) {   // piece i: token i / 6, 16 bytes i % 6 = (term, row tile)
+        const int i = i0 + lane, tok = i / 6 < 15 ? i / 6 : 15, part = i - 6 * (i / 6);
+        uint8_t* rec = rec_of(tok);
+        if (i < 96 && tok < nlive)
+            *reinterpret_cast<uint4*>(rec + 128 * (part >> 1) + 64 * (b & 1) + 32 * (part & 1) + 16 * (b >> 1)) =
+                *reinterpret_cast<const uint4*>(ls + tok * MXH_REC + 16 * part);
+    }
+    {
+        const int tok = lane & 15, t = lane >> 4;
+        uint8_t* rec = rec_of(tok);
+        if (t < 3 && tok < nlive) rec[384 + 4 * t + b] = ls[tok * MXH_REC + 96 + t];
+    }
+    if (pad) {   // wave-uniform. lane: token lane & 15, piece lane >> 4 of each term's blocks 2, 3
+        const int tok = lane & 15, bz = 2 + (lane >> 5), half = (lane >> 4) & 1;
+        uint8_t* rec = rec_of(tok);
+        if (tok < nlive)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                *reinterpret_cast<uint4*>(rec + 128 * t + 64 * (bz & 1) + 16 * (bz >> 1) + 32 * half) = uint4{0u, 0u, 0u, 0u};
+                if (!half) rec[384 + 4 * t + bz] = 127;
+            }
     }
 }
 
@@ -872,24 +888,27 @@ __global__ void __launch_bounds__(64) k_wave_tile(TileArgs a) {
             if (a.hterm) {
                 const int nslN = (N + 127) >> 7, bk = (r0 & 127) >> 5;
                 const bool pad = (N & 127) == 64 && (r0 >> 7) == nslN - 1 && bk == 1;
+                __shared__ __attribute__((aligned(16))) uint8_t sH[16 * MXH_REC];
+                float bg[RT], bu[RT];
 #pragma unroll
-                for (int t = 0; t < NT; ++t)
+                for (int rt = 0; rt < RT; ++rt) {
+                    const size_t r = (size_t)e * N + r0 + 16 * rt + lr;
+                    bg[rt] = a.b0 ? a.b0[r] : 0.f;
+                    bu[rt] = a.b1 ? a.b1[r] : 0.f;
+                }
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        const int j = 4 * lg + v;
-                        const int slot = __shfl(slotA[t], j, 64);   // lane j (any lane group) holds token j's slot
                         float hv[RT];
 #pragma unroll
-                        for (int rt = 0; rt < RT; ++rt) {
-                            const int r = r0 + 16 * rt + lr;
-                            float g = acc[0][rt][t][v], up = acc[1][rt][t][v];
-                            if (a.b0) g += a.b0[(size_t)e * N + r];
-                            if (a.b1) up += a.b1[(size_t)e * N + r];
-                            hv[rt] = glu_act(a.act, g, up);
-                        }
-                        mx_h_block<3>(hv[0], hv[1], tok0 + 16 * t + j < n,
-                                      a.hterm + ((size_t)slot * nslN + (r0 >> 7)) * mx_rec<3>(), bk, lr, pad);
+                        for (int rt = 0; rt < RT; ++rt)
+                            hv[rt] = glu_fast(a.act, acc[0][rt][t][v] + bg[rt], acc[1][rt][t][v] + bu[rt]);
+                        mx_h_terms(hv[0], hv[1], sH + (4 * lg + v) * MXH_REC, lr);
                     }
+                    mx_h_store(sH, n - tok0 - 16 * t, [&](int tok) { return __shfl(slotA[t], tok, 64); }, a.hterm, nslN, r0 >> 7,
+                               bk, pad);
+                }
                 return;
             }
         }
@@ -1215,36 +1234,31 @@ __global__ void __launch_bounds__(256) k_mx_terms(const uint16_t* __restrict__ s
 }
 
 // k_mxd: blocks of 4 waves own BN = 64 RT rows of one expert (per projection) and one pass of up to 64 of its slots
-// (the dense tiles' work list, XCD-chunked the same way); each wave covers the pass's 4 token tiles for its RT row
-// tiles. Per 128-input slice: the pass's activation records (64 x REC bytes) come into LDS by
-// global_load_lds_dwordx4 (records of 17 or 25 16-byte pieces, an odd count, so the 16 lanes of a token tile read
-// 16 distinct bank groups), double-buffered; each wave loads its row tiles' slice records (1 KB of codes + the
-// E8M0 words) one slice ahead; NTERM x 4 x NPROJ x RT MFMAs per slice.
-#ifndef MOE_MXD_RT_DN
-#define MOE_MXD_RT_DN 4
-#endif
-#ifndef MOE_MXD_MINB_GU
-#define MOE_MXD_MINB_GU 2
-#endif
-#ifndef MOE_MXD_MINB_DN
-#define MOE_MXD_MINB_DN 2
-#endif
+// (the dense tiles' work list, XCD-chunked the same way); each wave covers the pass's token tiles for its RT row
+// tiles. Per 128-input slice: the pass's activation records (64 x REC bytes) come into LDS by DMA (records of 17 or 25
+// 16-byte pieces, an odd count, so the 16 lanes of a token tile read 16 distinct bank groups), double-buffered; each wave
+// loads its row tiles' slice records (1 KB of codes + the E8M0 words) one slice ahead; NTERM x 4 x NPROJ x RT MFMAs per
+// slice, in steps of one (token tile, term): the next step's A operand is read from LDS while a step's MFMAs run. Buffer
+// addressing and the order of the prologue as in k_dense_i4.
 template <int NPROJ>
-__host__ __device__ constexpr int mxd_rt() { return NPROJ == 2 ? 2 : MOE_MXD_RT_DN; }
+__host__ __device__ constexpr int mxd_rt() { return 4 / NPROJ; }
 
 template <int NPROJ, int NTERM>
-__global__ void __launch_bounds__(256, NPROJ == 2 ? MOE_MXD_MINB_GU : MOE_MXD_MINB_DN) k_mxd(TileArgs a) {
-    constexpr int NT = 4, BM = 64;
+__global__ void __launch_bounds__(256, 3) k_mxd(TileArgs a) {
+#ifdef __HIP_DEVICE_COMPILE__
+    constexpr int BM = 64;
     constexpr int RT = mxd_rt<NPROJ>();
+    constexpr int CT = NPROJ * RT;
     constexpr int BN = 64 * RT;
     constexpr int REC = mx_rec<NTERM>();
     constexpr int NPC = REC / 16;                     // 16-byte pieces per record
     constexpr int NCH = (BM * NPC + 63) / 64;         // 64-piece DMA chunks per slice
     constexpr int NDMA = (NCH + 3) / 4;               // DMA instructions per wave per slice (the last partial)
+    constexpr int SB = TILE_SLICE_MXFP4;
     typedef int v8i __attribute__((ext_vector_type(8)));
     __shared__ __attribute__((aligned(1024))) uint8_t sX0[NCH * 1024];
     __shared__ __attribute__((aligned(1024))) uint8_t sX1[NCH * 1024];
-    __shared__ int sSlot[BM];
+    __shared__ __attribute__((aligned(16))) int sSlot[BM];
 
     const int nrb = (a.N + BN - 1) / BN;
     const int nitems = a.meta[a.nidx] * nrb;
@@ -1257,171 +1271,172 @@ __global__ void __launch_bounds__(256, NPROJ == 2 ? MOE_MXD_MINB_GU : MOE_MXD_MI
     const int w0 = wq - a.items[3 * wq + 1];
     const int local = item - w0 * nrb;
     const int rb = local / np;
-    const int n = a.counts[e], beg = a.offsets[e];
-    int tok0, nlive;
-    pass_tokens(n, np, local - rb * np, tok0, nlive);
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int K = a.K, N = a.N;
     const int nsl = (K + 127) >> 7;
     const int r0 = rb * BN + wave * 16 * RT;
     const bool wvalid = r0 < N;                        // N % (16 RT) == 0
-    constexpr int SB = TILE_SLICE_MXFP4;
-    const uint8_t* tb[NPROJ][RT];
+    const uint32_t trec = (uint32_t)nsl * SB;          // one 16-row tile's records
+    __amdgpu_buffer_rsrc_t wb[NPROJ];
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p)
+        wb[p] = buffer_of((p ? a.W1 : a.W0) + ((size_t)e * (N >> 4) + (wvalid ? (r0 >> 4) : 0)) * (size_t)trec, RT * trec);
+    const uint32_t wofs = 16u * lane, mofs = 1024u + 4u * lr;
+    // weights of slice s: the lane's 16 bytes of each row tile's record and its row's E8M0 word (words and groups
+    // past K are zero in the records: zero codes, scale 2^-127)
+    struct WS { u32x4 q[CT]; uint32_t m[CT]; };
+    auto fetch_w = [&](int s, WS& w) __attribute__((always_inline)) {
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-            tb[p][rt] = (p ? a.W1 : a.W0) + ((size_t)e * (N >> 4) + (wvalid ? (r0 >> 4) + rt : 0)) * (size_t)nsl * SB;
-    const uint8_t* recs = reinterpret_cast<const uint8_t*>(a.actv);
-
+        for (int c = 0; c < CT; ++c) {
+            const int so = (c % RT) * (int)trec + s * SB;
+            w.q[c] = __builtin_amdgcn_raw_buffer_load_b128(wb[c / RT], wofs, so, 0);
+            w.m[c] = __builtin_amdgcn_raw_buffer_load_b32(wb[c / RT], mofs, so, 0);
+        }
+    };
+    WS wa, wn;
+    fetch_w(0, wa);                                    // in flight while the pass's tokens are looked up
+    const int n = a.counts[e], beg = a.offsets[e];
+    int tok0, nlive;
+    pass_tokens(n, np, local - rb * np, tok0, nlive);
     const int ntiles = (nlive + 15) >> 4;
     if (tid < BM) sSlot[tid] = a.sorted[beg + (tok0 + tid < n ? tok0 + tid : n - 1)];
     __syncthreads();
-    // DMA lanes: chunk c = 4 i + wave of the slice's BM * NPC pieces; piece q = 64 c + lane -> record of token
-    // q / NPC, piece q % NPC (pieces past the last record re-read the last piece into the buffer's tail)
+    const __amdgpu_buffer_rsrc_t xb = buffer_of(a.actv, 0xFFFFFFFFu);
+    // DMA lanes: chunk c = 4 i + wave (at most NCH - 1: waves past it repeat the last chunk) of the slice's BM * NPC pieces;
+    // piece q = 64 c + lane -> record of token q / NPC, piece q % NPC (pieces past the last record re-read the last piece
+    // into the buffer's tail)
+    auto chunk_of = [&](int i) __attribute__((always_inline)) { return 4 * i + wave < NCH ? 4 * i + wave : NCH - 1; };
     uint32_t xoff[NDMA];
 #pragma unroll
     for (int i = 0; i < NDMA; ++i) {
-        int q = 64 * (4 * i + wave) + lane;
+        int q = 64 * chunk_of(i) + lane;
         q = q < BM * NPC ? q : BM * NPC - 1;
         const int tok = q / NPC, pc = q - tok * NPC;
         xoff[i] = ((uint32_t)(sSlot[tok] / a.act_div) * (uint32_t)nsl) * (uint32_t)REC + 16u * (uint32_t)pc;
     }
-    auto dma = [&](int s, uint8_t* buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < NDMA; ++i)
-            if (4 * i + wave < NCH) {   // wave-uniform
-                uint32_t o = xoff[i] + (uint32_t)s * (uint32_t)REC;
-                asm volatile("" : "+v"(o));
-                __builtin_amdgcn_global_load_lds((const void*)(recs + o), MOE_LDSP(buf + (4 * i + wave) * 1024), 16, 0, 0);
-            }
-    };
-    // weights of slice s: the lane's 16 bytes of each row tile's record and its row's E8M0 word (words and groups
-    // past K are zero in the records: zero codes, scale 2^-127)
-    auto wissue = [&](int s, uint4 (&q)[NPROJ][RT], uint32_t (&m)[NPROJ][RT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const uint8_t* sl = tb[p][rt] + (uint32_t)s * (uint32_t)SB;
-                q[p][rt] = *reinterpret_cast<const uint4*>(sl + 16 * lane);
-                m[p][rt] = *reinterpret_cast<const uint32_t*>(sl + 1024 + 4 * lr);
-            }
-    };
     // lane group g: words (g, 4 + g, 8 + g, 12 + g) -> (4 g, 4 g + 1, 4 g + 2, 4 g + 3)
-    auto transpose = [](const uint4& v) __attribute__((always_inline)) {
+    auto transpose = [](const u32x4& v) __attribute__((always_inline)) {
         const auto s0 = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
         const auto s1 = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
         const auto t0 = __builtin_amdgcn_permlane16_swap(s0[0], s1[0], false, false);
         const auto t1 = __builtin_amdgcn_permlane16_swap(s0[1], s1[1], false, false);
-        return uint4{t0[0], t0[1], t1[0], t1[1]};
+        return v8i{(int)t0[0], (int)t0[1], (int)t1[0], (int)t1[1], 0, 0, 0, 0};
     };
-    f32x4 acc[NPROJ][RT][NT];
+    f32x4 acc[CT][BM / 16];
 #pragma unroll
-    for (int p = 0; p < NPROJ; ++p)
+    for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
+        for (int t = 0; t < BM / 16; ++t) acc[c][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto run = [&](auto ntl) __attribute__((always_inline)) {
+        constexpr int L = decltype(ntl)::value;        // live token tiles
+        constexpr int CHL = (16 * L * NPC + 63) / 64;  // their DMA chunks
+        auto fetch_x = [&](int s, uint8_t* buf) __attribute__((always_inline)) {
 #pragma unroll
-            for (int t = 0; t < NT; ++t) acc[p][rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // token tile by token tile (live tiles only): the tile's NTERM A operands from LDS, then its MFMAs
-    auto compute = [&](const uint8_t* xs, const uint4 (&q)[NPROJ][RT], const uint32_t (&m)[NPROJ][RT])
-                       __attribute__((always_inline)) {
-        v8i B[NPROJ][RT];
-        int sb[NPROJ][RT];
+            for (int i = 0; i < (CHL + 3) / 4; ++i)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(xb, MOE_LDSP(buf + chunk_of(i) * 1024), 16, xoff[i], s * REC, 0, 0);
+        };
+        auto compute = [&](const uint8_t* xs, const WS& w) __attribute__((always_inline)) {
+            const uint8_t* ra = xs + lr * REC;
+            v8i B[CT], A[2];
+            int sb[CT], sa[2];
+            auto load_a = [&](int st, v8i& A_, int& sa_) __attribute__((always_inline)) {   // step st: tile st / NTERM
+                const uint8_t* r = ra + 16 * (st / NTERM) * REC;
+                const int tm = st % NTERM;
+                const uint4 a0 = *reinterpret_cast<const uint4*>(r + 128 * tm + 32 * lg);
+                const uint4 a1 = *reinterpret_cast<const uint4*>(r + 128 * tm + 32 * lg + 16);
+                A_ = v8i{(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w, (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
+                sa_ = r[128 * NTERM + 4 * tm + lg];
+            };
+            __builtin_amdgcn_sched_barrier(0);
+            load_a(0, A[0], sa[0]);
 #pragma unroll
-        for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) {
-                const uint4 w = transpose(q[p][rt]);
-                B[p][rt] = v8i{(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
-                sb[p][rt] = (int)(m[p][rt] >> (8 * lg));
-            }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            if (t < ntiles) {   // wave-uniform
-                const uint8_t* ra = xs + (16 * t + lr) * REC;
-                v8i A[NTERM];
-                int sa[NTERM];
-#pragma unroll
-                for (int tm = 0; tm < NTERM; ++tm) {
-                    const uint4 a0 = *reinterpret_cast<const uint4*>(ra + 128 * tm + 32 * lg);
-                    const uint4 a1 = *reinterpret_cast<const uint4*>(ra + 128 * tm + 32 * lg + 16);
-                    A[tm] = v8i{(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w, (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
-                    sa[tm] = ra[128 * NTERM + 4 * tm + lg];
-                }
-#pragma unroll
-                for (int tm = 0; tm < NTERM; ++tm)
-#pragma unroll
-                    for (int p = 0; p < NPROJ; ++p)
-#pragma unroll
-                        for (int rt = 0; rt < RT; ++rt)
-                            acc[p][rt][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                                A[tm], B[p][rt], acc[p][rt][t], 0, 4, 0, sa[tm], 0, sb[p][rt]);
+            for (int c = 0; c < CT; ++c) {
+                B[c] = transpose(w.q[c]);
+                sb[c] = (int)(w.m[c] >> (8 * lg));
             }
             __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int st = 0; st < L * NTERM; ++st) {
+                if (st + 1 < L * NTERM) load_a(st + 1, A[(st + 1) & 1], sa[(st + 1) & 1]);
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+                    acc[c][st / NTERM] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                        A[st & 1], B[c], acc[c][st / NTERM], 0, 4, 0, sa[st & 1], 0, sb[c]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        // slice s in buffer / register set s & 1; slice s + 1 is fetched while slice s is multiplied (the last slice
+        // fetches itself again into the idle set: no branch around the loads)
+        fetch_x(0, sX0);
+        MOE_VMWAIT0();
+        MOE_BARRIER();
+        int j = 0;
+        for (; j + 2 <= nsl; j += 2) {
+            fetch_w(j + 1, wn);
+            fetch_x(j + 1, sX1);
+            compute(sX0, wa);
+            MOE_VMWAIT0();
+            MOE_BARRIER();
+            const int jn = j + 2 < nsl ? j + 2 : j + 1;
+            fetch_w(jn, wa);
+            fetch_x(jn, sX0);
+            compute(sX1, wn);
+            MOE_VMWAIT0();
+            MOE_BARRIER();
         }
+        if (j < nsl) compute(sX0, wa);   // odd count: the last slice is in buffer 0
     };
-    uint4 rq[2][NPROJ][RT];
-    uint32_t rm[2][NPROJ][RT];
-    // slice s in buffer / register set s & 1; slice s + 1 is fetched while slice s is multiplied (the last slice
-    // fetches itself again into the idle set: no branch around the loads)
-    dma(0, sX0);
-    wissue(0, rq[0], rm[0]);
-    MOE_VMWAIT0();
-    MOE_BARRIER();
-    int j = 0;
-    for (; j + 2 <= nsl; j += 2) {
-        wissue(j + 1, rq[1], rm[1]);
-        dma(j + 1, sX1);
-        compute(sX0, rq[0], rm[0]);
-        MOE_VMWAIT0();
-        MOE_BARRIER();
-        const int jn = j + 2 < nsl ? j + 2 : j + 1;
-        wissue(jn, rq[0], rm[0]);
-        dma(jn, sX0);
-        compute(sX1, rq[1], rm[1]);
-        MOE_VMWAIT0();
-        MOE_BARRIER();
-    }
-    if (j < nsl) compute(sX0, rq[0], rm[0]);   // odd count: the last slice is in buffer 0
+    if (ntiles == 1) run(std::integral_constant<int, 1>{});
+    else if (ntiles == 2) run(std::integral_constant<int, 2>{});
+    else if (ntiles == 3) run(std::integral_constant<int, 3>{});
+    else run(std::integral_constant<int, 4>{});
 
     // ---- epilogue: lane holds row r0 + 16 rt + lr of tokens tok0 + 16 t + 4 lg + v
-    if (!wvalid) return;
     if constexpr (NPROJ == 2) {   // h as the down's 3-term records: this wave's 32 rows = one block
         static_assert(RT == 2, "one 32-row block of h per wave");
+        static_assert(4 * 16 * MXH_REC <= NCH * 1024, "a tile of h records per wave in the first buffer");
+        MOE_BARRIER();            // every wave is done with the activation buffers
+        if (!wvalid) return;
+        uint8_t* ls = sX0 + wave * 16 * MXH_REC;
         const int nslN = (N + 127) >> 7, bk = (r0 & 127) >> 5;
         const bool pad = (N & 127) == 64 && (r0 >> 7) == nslN - 1 && bk == 1;
+        float bg[RT], bu[RT];
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+        for (int rt = 0; rt < RT; ++rt) {
+            const size_t r = (size_t)e * N + r0 + 16 * rt + lr;
+            bg[rt] = a.b0 ? a.b0[r] : 0.f;
+            bu[rt] = a.b1 ? a.b1[r] : 0.f;
+        }
+#pragma unroll
+        for (int t = 0; t < BM / 16; ++t) {
+            if (t >= ntiles) break;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int jt = 16 * t + 4 * lg + v;
-                const int slot = sSlot[jt];
                 float hv[RT];
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt) {
-                    const int r = r0 + 16 * rt + lr;
-                    float g = acc[0][rt][t][v], up = acc[1][rt][t][v];
-                    if (a.b0) g += a.b0[(size_t)e * N + r];
-                    if (a.b1) up += a.b1[(size_t)e * N + r];
-                    hv[rt] = glu_act(a.act, g, up);
-                }
-                mx_h_block<3>(hv[0], hv[1], jt < nlive, a.hterm + ((size_t)slot * nslN + (r0 >> 7)) * mx_rec<3>(), bk,
-                              lr, pad);
+                for (int rt = 0; rt < RT; ++rt) hv[rt] = glu_fast(a.act, acc[rt][t][v] + bg[rt], acc[RT + rt][t][v] + bu[rt]);
+                mx_h_terms(hv[0], hv[1], ls + (4 * lg + v) * MXH_REC, lr);
             }
+            mx_h_store(ls, nlive - 16 * t, [&](int tok) { return sSlot[16 * t + tok]; }, a.hterm, nslN, r0 >> 7, bk, pad);
+        }
         return;
     }
+    if (!wvalid) return;
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < BM / 16; ++t) {
+        if (t >= ntiles) break;
+        const int j0 = 16 * t + 4 * lg;
+        const int4 s4 = *reinterpret_cast<const int4*>(&sSlot[j0]);
+        const int sl[4] = {s4.x, s4.y, s4.z, s4.w};
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int jt = 16 * t + 4 * lg + v;
-            if (jt >= nlive) continue;
-            const int slot = sSlot[jt];
+            if (j0 + v >= nlive) continue;
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt) a.yp[(size_t)slot * N + r0 + 16 * rt + lr] = acc[0][rt][t][v];
+            for (int rt = 0; rt < RT; ++rt) a.yp[(size_t)sl[v] * N + r0 + 16 * rt + lr] = acc[rt][t][v];
         }
+    }
+#endif
 }
 
 template <int NPROJ, int NTERM>
