@@ -1237,17 +1237,13 @@ __global__ void __launch_bounds__(256) k_mx_terms(const uint16_t* __restrict__ s
 // (the dense tiles' work list, XCD-chunked the same way); each wave covers the pass's token tiles for its RT row
 // tiles. Per 128-input slice: the pass's activation records (64 x REC bytes) come into LDS by DMA (records of 17 or 25
 // 16-byte pieces, an odd count, so the 16 lanes of a token tile read 16 distinct bank groups), double-buffered; each wave
-// loads its row tiles' slice records (1 KB of codes + the E8M0 words) one slice ahead; NTERM x 4 x NPROJ x RT MFMAs per
+// loads its row tiles' slice records (1 KB of codes + the E8M0 words) one slice ahead; NTERM x 4 x NPROJ RT MFMAs per
 // slice, in steps of one (token tile, term): the next step's A operand is read from LDS while a step's MFMAs run. Buffer
 // addressing and the order of the prologue as in k_dense_i4.
-template <int NPROJ>
-__host__ __device__ constexpr int mxd_rt() { return 4 / NPROJ; }
-
-template <int NPROJ, int NTERM>
+template <int NPROJ, int NTERM, int RT>
 __global__ void __launch_bounds__(256, 3) k_mxd(TileArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__
     constexpr int BM = 64;
-    constexpr int RT = mxd_rt<NPROJ>();
     constexpr int CT = NPROJ * RT;
     constexpr int BN = 64 * RT;
     constexpr int REC = mx_rec<NTERM>();
@@ -1439,13 +1435,13 @@ __global__ void __launch_bounds__(256, 3) k_mxd(TileArgs a) {
 #endif
 }
 
-template <int NPROJ, int NTERM>
+template <int NPROJ, int NTERM, int RT>
 int launch_mxd(const TileArgs& t, int nslots, hipStream_t st) {
-    constexpr int BN = 64 * mxd_rt<NPROJ>();
-    if (t.N % (16 * mxd_rt<NPROJ>())) return MOE_ERR_ARG;
+    constexpr int BN = 64 * RT;
+    if (t.N % (16 * RT)) return MOE_ERR_ARG;
     const long nblk = ((long)((t.N + BN - 1) / BN) * max_passes(nslots, t.E, 64) + 7) / 8 * 8;
     if (nblk > 0x7FFFFFF8L) return MOE_ERR_ARG;
-    k_mxd<NPROJ, NTERM><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
+    k_mxd<NPROJ, NTERM, RT><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
@@ -1822,7 +1818,20 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
     constexpr int BN_GU = dense_bn<FMT, 2>(), BN_DN = dense_bn<FMT, 1>();
     const long dblocks = (long)((w->F + BN_GU - 1) / BN_GU) * max_passes(nslots, w->E, DP);
     const long dn_blocks = (long)((w->d + BN_DN - 1) / BN_DN) * max_passes(nslots, w->E, DP);
-    const int min_avg = env_int("MOE_DENSE_MIN_AVG", 32);
+    // MXFP4 with bf16 x: the block-scaled MFMA kernels (MOE_MXMFMA=0: the bf16-MFMA tiles). x's terms go to the x-planes
+    // region, h's terms to the yp planes the split down would use; both must fit there, with 32-bit record offsets
+    const size_t mx_xb = (size_t)T * ((w->d + 127) / 128) * mx_rec<2>();
+    const size_t mx_hb = (size_t)nslots * ((w->F + 127) / 128) * mx_rec<3>();
+    const bool mx_fit = !INT4 && nx == 1 && env_int("MOE_MXMFMA", 1) && mx_xb <= (size_t)6 * T * w->d &&
+                        mx_hb <= (size_t)12 * nslots * w->d && mx_hb < (1ull << 32);
+    // slots per expert above which both stages run the dense tiles. MXFP4 with bf16 x (block-scaled MFMA, the same terms and
+    // sums in the wave and the dense tiles): from 11, if the down's 256-row blocks give every CU one, else from 15. Layers,
+    // wave / dense: gpt-oss T = 64 (8 slots per expert) 108.0 / 102.5 us, Zipf 107.3 / 111.8, T = 110 (14) Zipf 135.8 / 131.6,
+    // T = 192 (24) 187.7 / 126.7; OLMoE shape T = 70 (9) Zipf 64.8 / 66.2, T = 240 (30) 132.8 / 82.0; Qwen3 shape T = 128 (8)
+    // 92.9 / 90.5; few blocks: Mixtral shape T = 40 (10) 178 / 209, T = 70 (18) 243 / 218; d = 1088, E = 40 T = 200 (15)
+    // 36.8 / 35.9. The other formats and dtypes: from 33.
+    const long mx_dn_blocks = (long)((w->d + 255) / 256) * (nslots < w->E ? nslots : w->E);
+    const int min_avg = env_int("MOE_DENSE_MIN_AVG", !mx_fit ? 32 : mx_dn_blocks >= 256 ? 10 : 14);
     const int dn_min_avg = env_int("MOE_DENSE_DN_MIN_AVG", 16);
     // activations as planes (fp16 / fp32 x): the dense gate/up takes only what it reads exactly, int4 with fp16 x
     // (x16); fp32 x and MXFP4 keep the exact-operand wave / row tiles, one 16-token tile per pass (nt = 1: the
@@ -1832,16 +1841,9 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
                  (dmode == 1 || (dmode < 0 && dblocks >= MOE_DENSE_MIN_BLOCKS));
     p.dense_dn = p.dense_gu || (INT4 && p.tiled && dmode != 0 && avg > dn_min_avg &&
                                 (dmode == 1 || dn_blocks >= MOE_DENSE_MIN_BLOCKS));
-    // MXFP4 with bf16 x on the dense tiles: the block-scaled MFMA kernels instead (MOE_MXMFMA=0: the bf16-MFMA
-    // dense tiles). x's terms go to the x-planes region, h's terms to the yp planes the split down would use; both
-    // must fit there, with 32-bit record offsets
-    const size_t mx_xb = (size_t)T * ((w->d + 127) / 128) * mx_rec<2>();
-    const size_t mx_hb = (size_t)nslots * ((w->F + 127) / 128) * mx_rec<3>();
-    const bool mx_fit = !INT4 && nx == 1 && env_int("MOE_MXMFMA", 1) && mx_xb <= (size_t)6 * T * w->d &&
-                        mx_hb <= (size_t)12 * nslots * w->d && mx_hb < (1ull << 32);
-    p.mxd = mx_fit && p.dense_gu && w->F % (16 * mxd_rt<2>()) == 0 && w->d % (16 * mxd_rt<1>()) == 0;
-    p.wave_gu = p.tiled && !p.dense_gu && (avg <= min_avg || dmode != 0);
-    p.wave_dn = p.tiled && !p.dense_dn && (avg <= min_avg || dmode != 0);
+    p.mxd = mx_fit && p.dense_gu && w->F % 32 == 0 && w->d % 64 == 0;
+    p.wave_gu = p.tiled && !p.dense_gu && (avg <= 32 || dmode != 0);
+    p.wave_dn = p.tiled && !p.dense_dn && (avg <= 32 || dmode != 0);
     // the wave tiles of MXFP4 with bf16 x on the block-scaled MFMA too (terms as for the dense kernels)
     p.mxw = mx_fit && p.wave_gu && p.wave_dn;
     p.h16 = INT4 && p.dense_dn;   // h leaves the gate/up as h16 with per-32-row exponents
@@ -1941,7 +1943,7 @@ int run_tiles_fmt(const ExpertsArgs& a) {
             g.W1 = (const uint8_t*)w->up.tiles;
             if (!a.xterm_ready) rc = launch_mx_terms<2>(a.xb, a.T, w->d, a.xterm, a.st);
             g.actv = reinterpret_cast<const uint16_t*>(a.xterm);
-            if (!rc) rc = launch_mxd<2, 2>(g, nslots, a.st);
+            if (!rc) rc = launch_mxd<2, 2, 2>(g, nslots, a.st);
             if (rc) return rc;
         } else if (dense_gu && INT4) {
             if (a.x_dtype == MOE_DTYPE_F16) k_x16<MOE_DTYPE_F16><<<a.T, 256, 0, a.st>>>(a.x, a.x16, a.xexp, w->d);
@@ -2002,7 +2004,11 @@ int run_tiles_fmt(const ExpertsArgs& a) {
         const int mxt = mxw ? 3 : 0;
         if (mxd) {
             d.W0 = (const uint8_t*)w->down.tiles;
-            rc = launch_mxd<1, 3>(d, nslots, a.st);
+            // 64 rows per wave (each A operand feeds four MFMAs) once that gives two blocks per CU, else 32: gpt-oss T = 192
+            // (528 blocks) 126.7 / 130.8 us per layer, T = 160 Zipf (504) 146.4 / 140.9, Mixtral shape T = 70 (176) 228 / 218,
+            // T = 300 (288) 340 / 328, OLMoE shape T = 240 (752) 82.0 / 88.5
+            const long blocks = (long)((d.N + 255) / 256) * max_passes(nslots, w->E, 64);
+            rc = blocks >= 512 ? launch_mxd<1, 3, 4>(d, nslots, a.st) : launch_mxd<1, 3, 2>(d, nslots, a.st);
         } else if (dense_dn) {
             // int4: 32 rows per wave at four blocks per CU; 64 rows (three blocks) or 32-token tiles measured slower on
             // every shape but Qwen3 T = 4096 (even)

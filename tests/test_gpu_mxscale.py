@@ -205,3 +205,23 @@ def test_mxscale_wave_stages_split_and_ingroup(monkeypatch):
     torch.cuda.synchronize()
     assert torch.equal(y, y2)
     assert torch.equal(y, y3)
+
+
+@pytest.mark.parametrize("counts", [[11, 12, 15, 16, 17, 1, 33, 31], [64, 65, 63, 128, 129, 16, 0, 1]])
+@pytest.mark.parametrize("d,F", [(128, 64), (320, 192), (2880, 64)])
+def test_dense_from_eleven_slots_token_tile_edges(monkeypatch, counts, d, F):
+    """The block-scaled dense tiles at the loads they now take (11 slots per expert and up): counts around multiples of a
+    token tile and of a pass, row blocks partly past N, a K that ends at half a slice, records assembled in LDS."""
+    from moelab_amd import _lib, experts
+    from moelab_amd.problem import baseline_mxfp4_layer
+    from moelab_amd.shapes import MoEShape
+    monkeypatch.setenv("MOE_DENSE", "1")
+    E, T = len(counts), sum(counts)
+    s = baseline_mxfp4_layer(MoEShape("t", d=d, f=F, E=E, k=1), seed=T + d, device=DEV, router=False)
+    rng = np.random.default_rng(T)
+    idx = torch.from_numpy(rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts))[:, None].copy()).to(DEV)
+    wts = torch.from_numpy(rng.random((T, 1), dtype=np.float32)).to(DEV)
+    x = torch.from_numpy(rng.standard_normal((T, d), dtype=np.float32)).to(DEV).to(torch.bfloat16)
+    print(f"case mx dense d={d} F={F} counts={counts}", flush=True)
+    y = experts.run_experts(s, x, idx, wts, act=2, path=_lib.PATH_GROUPED, out_dtype=torch.float32)
+    assert_close(y, oracle_y(s, x, idx, wts, act=2), tol=2e-3, what=(d, F, counts))   # the file's bound
