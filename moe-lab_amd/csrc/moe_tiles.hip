@@ -1519,68 +1519,58 @@ __global__ void __launch_bounds__(256) k_x16(const void* __restrict__ x, uint16_
     }
 }
 
-// int4 grouped path, between gate/up and a dense down: one block per slot. The gate/up wrote h16 = h 2^-e with e
-// per (slot, 32-row chunk) (h16_exponent); this brings the slot's row to one exponent E = max e (chunks with a
-// smaller e are scaled by 2^(e - E): exact unless a value falls into fp16's subnormal range, where it is rounded:
-// it is then below 2^-24 of the slot's largest) and writes E for the down projection's epilogue. All-zero chunks
-// (H16_ZERO_EXP) take no part. A slot whose chunks share one exponent (the usual case: all 0) costs two exponent
-// loads per thread.
+// int4 grouped path, between gate/up and a dense down. The gate/up wrote h16 = h 2^-e with e per (slot, 32-row chunk)
+// (h16_exponent); this brings a slot's row to one exponent E = max e (chunks with a smaller e are scaled by 2^(e - E):
+// exact unless a value falls into fp16's subnormal range, where it is rounded: it is then below 2^-24 of the slot's
+// largest) and writes E for the down projection's epilogue. All-zero chunks (H16_ZERO_EXP) take no part. LPS lanes
+// read a slot's exponent bytes; a slot whose chunks share one exponent (the usual case: all 0) needs nothing more, the others
+// are rewritten by the whole wave, one after another. LPS lanes per slot: 8, or the whole wave from F = 4096 (8 lanes read
+// 448 chunks of F = 14336 in 8.7 us, a workgroup per slot in 4.8). Bound: the exponent bytes' latency and, in a large call,
+// workgroup dispatch: with a workgroup per slot 24 us at 32768 slots of F = 768, 5.0 us now.
+template <int LPS>
 __global__ void __launch_bounds__(256) k_h16_fix(const int8_t* __restrict__ hexp, uint16_t* __restrict__ h16,
-                                                 int32_t* __restrict__ eslot, int F) {
-    __shared__ int sE[512];   // F <= 16384: at most 512 chunks of 32
-    __shared__ int sMax[4], sMin[4];
-    const int slot = blockIdx.x, tid = threadIdx.x, nch = F >> 5;
-    const int8_t* er = hexp + (size_t)slot * nch;
-    const int e0 = tid < nch ? er[tid] : H16_ZERO_EXP, e1 = tid + 256 < nch ? er[tid + 256] : H16_ZERO_EXP;
-    sE[tid] = e0;
-    sE[tid + 256] = e1;
-    int m = e0 > e1 ? e0 : e1;
-    const int n0 = e0 == H16_ZERO_EXP ? 127 : e0, n1 = e1 == H16_ZERO_EXP ? 127 : e1;
-    int mn = n0 < n1 ? n0 : n1;
-    for (int o = 32; o; o >>= 1) {
-        const int other = __shfl_xor(m, o, 64), omn = __shfl_xor(mn, o, 64);
-        m = other > m ? other : m;
-        mn = omn < mn ? omn : mn;
-    }
-    if ((tid & 63) == 0) {
-        sMax[tid >> 6] = m;
-        sMin[tid >> 6] = mn;
-    }
-    __syncthreads();
-    int E = sMax[0];
-    mn = sMin[0];
-    for (int w = 1; w < 4; ++w) {
-        E = sMax[w] > E ? sMax[w] : E;
-        mn = sMin[w] < mn ? sMin[w] : mn;
-    }
-    if (tid == 0) eslot[slot] = E == H16_ZERO_EXP ? 0 : E;
-    if (mn >= E) return;   // block-uniform: every chunk with a non-zero value is at E already (or none has one)
-    // 16-byte pieces (8 values; 4 per chunk) of the row: every load first, then the rewrites
-    constexpr int CPT = 8;   // pieces per thread per round (F <= 16384: 2048 pieces, one round)
-    uint4* row = reinterpret_cast<uint4*>(h16 + (size_t)slot * F);
-    const int np = F >> 3;
-    for (int c0 = 0; c0 < np; c0 += 256 * CPT) {
-        uint4 v[CPT];
+                                                 int32_t* __restrict__ eslot, int F, int nslots) {
+    constexpr int SPW = 64 / LPS;   // slots per wave
+    const int lane = threadIdx.x & 63, ll = lane % LPS, nch = F >> 5;   // nch is even (F % 64 == 0)
+    const int slot0 = (blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * SPW, slot = slot0 + lane / LPS;
+    int m = H16_ZERO_EXP, mn = 127;
+    if (slot < nslots) {
+        const uint16_t* er = reinterpret_cast<const uint16_t*>(hexp + (size_t)slot * nch);
+        for (int c = ll; c < nch >> 1; c += LPS) {
+            const uint32_t v = er[c];
 #pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            const int c = c0 + i * 256 + tid;
-            if (c < np) v[i] = row[c];
+            for (int i = 0; i < 2; ++i) {
+                const int e = (int8_t)(v >> (8 * i));
+                m = e > m ? e : m;
+                if (e != H16_ZERO_EXP) mn = e < mn ? e : mn;
+            }
         }
+    }
 #pragma unroll
-        for (int i = 0; i < CPT; ++i) {
-            const int c = c0 + i * 256 + tid;
-            if (c >= np) continue;
-            const int ec = sE[c >> 2];
+    for (int o = 1; o < LPS; o <<= 1) {
+        const int om = __shfl_xor(m, o, 64), on = __shfl_xor(mn, o, 64);
+        m = om > m ? om : m;
+        mn = on < mn ? on : mn;
+    }
+    if (slot < nslots && ll == 0) eslot[slot] = m == H16_ZERO_EXP ? 0 : m;
+    uint64_t todo = __ballot(ll == 0 && mn < m);   // slots with chunks at different exponents
+    while (todo) {
+        const int src = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const int E = __builtin_amdgcn_readlane(m, src), s = slot0 + src / LPS;
+        uint4* row = reinterpret_cast<uint4*>(h16 + (size_t)s * F);
+        for (int c = lane; c < F >> 3; c += 64) {   // 16-byte pieces: 8 values, 4 per chunk
+            const int ec = hexp[(size_t)s * nch + (c >> 2)];
             if (ec == E || ec == H16_ZERO_EXP) continue;
-            const int d = ec - E;
-            uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+            const uint4 v = row[c];
+            uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 uint32_t out = 0;
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const float f = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[q] >> (16 * h)));
-                    out |= (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__builtin_ldexpf(f, d)) << (16 * h);
+                    out |= (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__builtin_ldexpf(f, ec - E)) << (16 * h);
                 }
                 w[q] = out;
             }
@@ -1968,8 +1958,10 @@ int run_tiles_fmt(const ExpertsArgs& a) {
         else if (wave_gu) rc = launch_wave_tile<FMT, 2, MOE_WAVE_RT_GU, MOE_WAVE_D_GU>(g, nt, nslots, a.st, a.nx);
         else rc = launch_tile<FMT, 2>(g, nt, max_active, a.T, a.st, a.nx);
         if (!rc && h16) {
-            k_h16_fix<<<nslots, 256, 0, a.st>>>((const int8_t*)a.hlo, a.hhi,
-                                              (int32_t*)((uint8_t*)a.hlo + t.eslot_off), w->F);
+            const int8_t* he = (const int8_t*)a.hlo;
+            int32_t* es = (int32_t*)((uint8_t*)a.hlo + t.eslot_off);
+            if (w->F >= 4096) k_h16_fix<64><<<(nslots + 3) / 4, 256, 0, a.st>>>(he, a.hhi, es, w->F, nslots);
+            else k_h16_fix<8><<<(nslots + 31) / 32, 256, 0, a.st>>>(he, a.hhi, es, w->F, nslots);
             rc = hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
         }
         if (rc) return rc;

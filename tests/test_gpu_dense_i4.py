@@ -54,3 +54,27 @@ def test_dead_tokens_and_large_h_write_only_their_slots(monkeypatch):
     want = oracle_y(s, x, idx, wts)
     for rows in (slice(0, None, 7), slice(3, None, 7), slice(1, None, 7)):
         assert_close(y[rows], want[rows], tol=1e-2, what=rows)
+
+
+@pytest.mark.parametrize("F", [64, 192, 1088, 4096])   # 4096: a wave per slot
+def test_slot_exponents_brought_together(monkeypatch, F):
+    """Slots whose 32-row chunks need different exponents (W_up rows at very different scales), mixed with slots that need
+    none and zero rows, over more slots than one workgroup takes, the last one partly filled."""
+    from moelab_amd import _lib, experts, formats
+    monkeypatch.setenv("MOE_DENSE", "1")
+    d, E, T = 128, 2, 137
+    g = torch.Generator(device=DEV).manual_seed(F)
+    gate, up, down = (formats.random_int4(E, n, k, generator=g, device=DEV) for n, k in ((F, d), (F, d), (d, F)))
+    grow = torch.ones(F, device=DEV)
+    grow[:32] = 2.0 ** 14          # the first chunk of every h row far above the others
+    up = (up[0], (up[1].float() * grow[None, :, None]).to(torch.bfloat16), (up[2].float() * grow[None, :, None]).to(torch.bfloat16))
+    s = experts.make_state("int4", gate, up, down)
+    x = torch.randn((T, d), generator=g, device=DEV).to(torch.bfloat16)
+    x[::5] *= 2.0 ** -12           # nothing to bring together here
+    x[7] = 0
+    idx = (torch.arange(T, device=DEV, dtype=torch.int32) % 2)[:, None].contiguous()
+    y = experts.run_experts(s, x, idx, torch.ones((T, 1), device=DEV), path=_lib.PATH_GROUPED, out_dtype=torch.float32)
+    want = oracle_y(s, x, idx, torch.ones((T, 1), device=DEV))
+    assert (y[7] == 0).all()
+    for rows in (slice(0, None, 5), slice(1, None, 5), slice(3, None, 5)):
+        assert_close(y[rows], want[rows], tol=5e-3, what=(F, rows))
