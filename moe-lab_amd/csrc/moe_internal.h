@@ -77,6 +77,7 @@ int launch_shared_route(const void* x, int xdt, const uint16_t* gate, int T, int
 struct TilePasses {
     int P, P2, ingroup;
     int mx;   // the call runs the block-scaled MXFP4 tiles, which read x as 2-term fp8 records (xterm)
+    int x16;  // the call's gate/up reads x as x16 (k_x16), not as bf16 planes
 };
 TilePasses tile_passes(const moe_experts_t* w, int T, int k, int x_dtype);
 

@@ -2028,7 +2028,8 @@ int run_experts_tiles(const ExpertsArgs& a) {
 
 TilePasses tile_passes(const moe_experts_t* w, int T, int k, int x_dtype) {
     const Plan p = w->fmt == MOE_FMT_INT4_G64 ? make_plan<FmtInt4>(w, T, k, x_dtype) : make_plan<FmtMxfp4>(w, T, k, x_dtype);
-    return TilePasses{p.P_gu, p.two_lists ? p.P_dn : 0, p.ingroup ? 1 : 0, p.mxd || p.mxw ? 1 : 0};
+    return TilePasses{p.P_gu, p.two_lists ? p.P_dn : 0, p.ingroup ? 1 : 0, p.mxd || p.mxw ? 1 : 0,
+                      w->fmt == MOE_FMT_INT4_G64 && p.dense_gu ? 1 : 0};
 }
 
 int launch_pack_tiles(int fmt, int E, int N, int K, const void* rows, void* tiles, hipStream_t st) {
