@@ -1,7 +1,7 @@
 // int4 dense tiles on fp16 MFMA (included by moe_tiles.hip after TileArgs): calls with many tokens per expert.
 #pragma once
 
-// A 4-wave block owns 128 RT rows of one expert (per projection) and one pass of up to 64 of its tokens, NT tiles of M;
+// A 4-wave block owns 128 RT rows of one expert (per projection) and one pass of up to BM of its tokens, NT tiles of M;
 // wave w takes 32 RT of the rows for all the pass's tokens, so each weight is decoded once per pass. Per 128-input slice
 // the tokens' activations (x16 / h16, fp16) come into LDS by DMA and the wave's weight records into registers, both one
 // slice ahead in two buffers; one wait and one barrier per slice.
@@ -16,10 +16,19 @@
 // Bound: decode and MFMA issue, then the chip's power: MFMAs alone on random data run at ~1.65 PFLOP/s here (1.6 GHz),
 // with 24 VALU per 128 MFMA cycles at ~1.5. Gate/up kernel, against the kernel before (16 x 16 tiles at 2 blocks per CU,
 // libm GLU, decode between whole steps): Mixtral T = 512 354 -> 294 us (820 TFLOP/s), Qwen3 T = 4096 320 -> 260.
-template <int NPROJ, int RT, int M, int MINB>
+//
+// EX (gate/up): products on exact weights, for loads where the wave tiles' exact codes were used before. The decode
+// takes s (q - 8) instead of s q + b: 8 + 3 significant bits, which fp16 holds exactly (below the subnormal line of the
+// row scaling: to 2^-22 of the row's largest), and what is left, sum over groups of (b + 8 s) XS with XS = the group's sum of
+// activations, is a product over groups of its own: one MFMA per GS = 4 (M = 16) or 2 slices and tile pair, lane group
+// g holding slice GS i + g, both factors as fp16 hi + lo (hi hi + lo hi + hi lo, 22 bits). k_x16 writes XS in A-operand form.
+// Against 64 bits the layer is then as far off as with the wave tiles (the fp16 rounding of h).
+template <int NPROJ, int RT, int M, int BM, int MINB, bool EX = false>
 __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__   // buffer resources exist in device code only
-    constexpr int BM = 64, NT = BM / M, BN = 128 * RT;
+    static_assert(!EX || NPROJ == 2, "exact weights: gate/up");
+    constexpr int NT = BM / M, BN = 128 * RT;
+    constexpr int GS = 64 / M;            // EX: slices per MFMA of the group-sum term
     constexpr int CT = NPROJ * RT;        // 32-row groups per wave
     constexpr int H = 32 / M;             // B tiles per group
     constexpr int CB = CT * H;
@@ -103,6 +112,11 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
 #pragma unroll
     for (int i = 0; i < BM / 16; ++i)
         xrow[i] = (uint32_t)(sSlot[4 * (wave + 4 * i) + (lane >> 4)] / a.act_div) * (uint32_t)K * 2u;
+    // EX: the lane's tokens' group sums (token ln of each tile), 16 bytes per slice
+    const __amdgpu_buffer_rsrc_t gb = buffer_of(a.xsum, 0xFFFFFFFFu);
+    uint32_t grow[EX ? NT : 1];
+#pragma unroll
+    for (int t = 0; t < (EX ? NT : 0); ++t) grow[t] = (uint32_t)(sSlot[M * t + ln] / a.act_div) * (uint32_t)nsl * 16u;
     // LDS offset of the lane's A operand of step 0; the later steps' words differ in the bits of 16 * word only
     uint32_t aofs = (uint32_t)ln * 256u + 16u * (((NJ / 2) * lg) ^ (ln & 15));
 
@@ -130,7 +144,7 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
 #pragma unroll
                 for (int b = 0; b < CB; ++b) {
                     const uint32_t mw = G ? w.m[b].y : w.m[b].x;
-                    const _Float16 s16 = (_Float16)(bf16lo(mw) * 16.0f), b16 = (_Float16)(bf16hi(mw) * 0x1p-16f);
+                    const _Float16 s16 = (_Float16)(bf16lo(mw) * 16.0f), b16 = (_Float16)(EX ? bf16lo(mw) * -0x1p-13f : bf16hi(mw) * 0x1p-16f);
                     s2[G][b] = h2x{s16, s16};
                     b2[G][b] = h2x{b16, b16};
                 }
@@ -192,6 +206,44 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
+        // EX: the group-sum term of slices s4 .. s4 + GS - 1 (s4 = GS i), loaded at slice s4, multiplied two slices later
+        f16x8 gx[EX ? L : 1];
+        u32x2 gm[EX ? CB : 1];
+        auto fetch_g = [&](int s4) __attribute__((always_inline)) {
+            if constexpr (EX) {
+                const int sl = s4 + lg < nsl ? s4 + lg : nsl - 1;
+#pragma unroll
+                for (int t = 0; t < L; ++t)
+                    gx[t] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(gb, grow[t] + 16u * sl, 0, 0));
+#pragma unroll
+                for (int b = 0; b < CB; ++b)
+                    gm[b] = __builtin_amdgcn_raw_buffer_load_b64(wb[b / (RT * H)], mofs + (uint32_t)(sl * SB),
+                                                                  (b % (RT * H)) * (2 / H) * (int)trec, 0);
+                if (s4 + lg >= nsl)
+#pragma unroll
+                    for (int b = 0; b < CB; ++b) gm[b] = u32x2{0u, 0u};
+            }
+        };
+        auto apply_g = [&]() __attribute__((always_inline)) {
+            if constexpr (EX) {
+#pragma unroll
+                for (int b = 0; b < CB; ++b) {
+                    _Float16 hi[2], lo[2];
+#pragma unroll
+                    for (int G = 0; G < 2; ++G) {   // (b + 8 s) 2^-16, times the 2^6 that XS is scaled down by
+                        const float v = __builtin_fmaf(8.f, bf16lo(gm[b][G]), bf16hi(gm[b][G])) * 0x1p-10f;
+                        hi[G] = (_Float16)v;
+                        lo[G] = (_Float16)(v - (float)hi[G]);
+                    }
+                    const f16x8 Bg = {hi[0], hi[1], lo[0], lo[1], hi[0], hi[1], (_Float16)0, (_Float16)0};
+#pragma unroll
+                    for (int t = 0; t < L; ++t) {
+                        if constexpr (M == 32) acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(gx[t], Bg, acc[b][t], 0, 0, 0);
+                        else acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(gx[t], Bg, acc[b][t], 0, 0, 0);
+                    }
+                }
+            }
+        };
         fetch_x(sb0, sX0);
         MOE_VMWAIT0();
         MOE_BARRIER();
@@ -199,6 +251,10 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
         for (; j + 2 <= scnt; j += 2) {
             fetch_w(sb0 + j + 1, wn);
             fetch_x(sb0 + j + 1, sX1);
+            if constexpr (EX) {
+                if (GS == 4 ? (j & 2) : j) apply_g();
+                if (GS == 2 || !(j & 2)) fetch_g(j);
+            }
             compute(sX0, wa);
             MOE_VMWAIT0();
             MOE_BARRIER();
@@ -209,13 +265,22 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
             MOE_VMWAIT0();
             MOE_BARRIER();
         }
+        if constexpr (EX) {   // the last group sums: fetched in the loop but not multiplied, or not fetched yet
+            if (GS == 4 ? (j & 2) : j) apply_g();
+            if ((GS == 2 || !(j & 2)) && j < scnt) {
+                fetch_g(j);
+                apply_g();
+            }
+        }
         if (j < scnt) compute(sX0, wa);   // odd count: the last slice is in buffer 0
     };
-    if (ntiles == 1) run(std::integral_constant<int, 1>{});
-    else if (ntiles == 2) run(std::integral_constant<int, 2>{});
-    else if constexpr (NT == 4) {
-        if (ntiles == 3) run(std::integral_constant<int, 3>{});
-        else run(std::integral_constant<int, 4>{});
+    if (NT == 1 || ntiles == 1) run(std::integral_constant<int, 1>{});
+    else if constexpr (NT >= 2) {
+        if (NT == 2 || ntiles == 2) run(std::integral_constant<int, 2>{});
+        else if constexpr (NT == 4) {
+            if (ntiles == 3) run(std::integral_constant<int, 3>{});
+            else run(std::integral_constant<int, 4>{});
+        }
     }
 
     // ---- epilogue: lane holds row r0 + M b + ln of tokens M t + (8 q) + 4 lg + v of the pass (v = 0..3, acc entry 4 q + v)

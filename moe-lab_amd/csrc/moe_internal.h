@@ -99,6 +99,7 @@ struct ExpertsArgs {
     float* yp;      // 4 x [T*k, d] fp32 scratch (grouped path; the further planes for a K-split down projection)
     uint16_t* x16;  // grouped path, dense int4: x as fp16 [T, d] with a power-of-two exponent per token
     int32_t* xexp;  // [T]
+    uint8_t* xsum;  // grouped path, dense int4 on exact weights: x16's group sums (the x-planes region: x16 is read instead)
     uint8_t* xterm; // grouped path, MXFP4 block-scaled MFMA: x's fp8 term records (the x-planes region when x is bf16)
     GroupBufs grp;  // grouped path
     int pregrouped; // grouped path: grp already holds the grouping and pass lists of idx (written by the router)

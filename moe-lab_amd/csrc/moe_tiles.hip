@@ -161,6 +161,7 @@ struct TileArgs {
     size_t plane;
     size_t eslot_off;      // dense int4 down: per-slot exponents (int32 [slots]) at this byte offset from the exponent bytes
     const int32_t* xexp;   // dense int4 gate/up: per-token exponents of x16 (actv) [T]
+    const uint8_t* xsum;   // dense int4 gate/up on exact weights: x16's group sums [T][ceil(K/128)][16 bytes]
     uint8_t* hterm;        // block-scaled MXFP4 gate/up: h leaves as 3-term records [T*k][ceil(N/128)] (no planes)
 };
 
@@ -1478,9 +1479,12 @@ __device__ __forceinline__ void load_x8(const void* row, int c, float v[8]) {
     }
 }
 
+// xsum (the exact-weight gate/up): also the sums of x16 over the 64-input groups, 16 bytes per token and 128-input slice in
+// A-operand form: XS 2^-6 of its two groups as fp16 hi + lo, (hi0, hi1, hi0, hi1, lo0, lo1, 0, 0). x16 then takes the
+// exponent that puts every row's largest at [2^14, 2^15), so that bf16 rows keep inputs down to 2^-38 of it.
 template <int XDT>
 __global__ void __launch_bounds__(256) k_x16(const void* __restrict__ x, uint16_t* __restrict__ x16,
-                                             int32_t* __restrict__ xexp, int d) {
+                                             int32_t* __restrict__ xexp, uint8_t* __restrict__ xsum, int d) {
     __shared__ float sM[4];
     const int t = blockIdx.x, tid = threadIdx.x;
     const void* row = reinterpret_cast<const uint8_t*>(x) + (size_t)t * d * (XDT == MOE_DTYPE_F32 ? 4 : 2);
@@ -1504,18 +1508,38 @@ __global__ void __launch_bounds__(256) k_x16(const void* __restrict__ x, uint16_
     if ((tid & 63) == 0) sM[tid >> 6] = am;
     __syncthreads();
     const float amax = fmaxf(fmaxf(sM[0], sM[1]), fmaxf(sM[2], sM[3]));
-    const int E = h16_exponent(amax);
+    int E = h16_exponent(amax);
+    if (xsum && E == 0 && amax == amax) {   // an ordinary row: the same rule as for the large and small ones
+        E = (int)((__float_as_uint(amax) >> 23) & 0xFFu) - 141;
+    }
     if (tid == 0) xexp[t] = E;
-    for (int c = tid; c < nch; c += 256) {   // the row again (cache hits)
-        float v[8];
-        load_x8<XDT>(row, c, v);
-        uint32_t o4[4];
+    for (int c0 = 0; c0 < nch; c0 += 256) {   // the row again (cache hits)
+        const int c = c0 + tid;
+        float sum = 0.f;
+        if (c < nch) {
+            float v[8];
+            load_x8<XDT>(row, c, v);
+            uint32_t o4[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const _Float16 lo = (_Float16)__builtin_ldexpf(v[2 * q], -E), hi = (_Float16)__builtin_ldexpf(v[2 * q + 1], -E);
-            o4[q] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
+            for (int q = 0; q < 4; ++q) {
+                const _Float16 lo = (_Float16)__builtin_ldexpf(v[2 * q], -E), hi = (_Float16)__builtin_ldexpf(v[2 * q + 1], -E);
+                o4[q] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
+                sum += (float)lo + (float)hi;
+            }
+            out[c] = make_uint4(o4[0], o4[1], o4[2], o4[3]);
         }
-        out[c] = make_uint4(o4[0], o4[1], o4[2], o4[3]);
+        if (xsum) {   // 8 chunks per group, 16 per slice; a slice that ends at input 64 has a zero second group
+            sum = sum_lanes<8>(sum);
+            const float s1 = __shfl(sum, (tid & 63) | 8, 64);
+            if (c < nch && (c & 15) == 0) {
+                const float w0 = sum * 0x1p-6f, w1 = s1 * 0x1p-6f;
+                const _Float16 h0 = (_Float16)w0, h1 = (_Float16)w1;
+                const _Float16 l0 = (_Float16)(w0 - (float)h0), l1 = (_Float16)(w1 - (float)h1);
+                const uint32_t hh = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
+                const uint32_t ll = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
+                reinterpret_cast<uint4*>(xsum)[(size_t)t * ((d + 127) >> 7) + (c >> 4)] = make_uint4(hh, hh, ll, 0u);
+            }
+        }
     }
 }
 
@@ -1768,14 +1792,14 @@ int launch_dense(TileArgs t, int nslots, hipStream_t st) {
     k_dense<NPROJ><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
-template <int NPROJ, int RT, int M, int MINB>
+template <int NPROJ, int RT, int M, int BM, int MINB, bool EX = false>
 int launch_dense_i4(TileArgs t, int nslots, hipStream_t st) {
     constexpr int BN = 128 * RT;
     if (t.N % (32 * RT)) return MOE_ERR_ARG;   // whole row tiles per wave
     if (NPROJ == 2) t.ksplit = 1;
-    const long nblk = ((long)((t.N + BN - 1) / BN) * max_passes(nslots, t.E, 64) * t.ksplit + 7) / 8 * 8;
+    const long nblk = ((long)((t.N + BN - 1) / BN) * max_passes(nslots, t.E, BM) * t.ksplit + 7) / 8 * 8;
     if (nblk > 0x7FFFFFF8L) return MOE_ERR_ARG;
-    k_dense_i4<NPROJ, RT, M, MINB><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
+    k_dense_i4<NPROJ, RT, M, BM, MINB, EX><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
@@ -1791,7 +1815,7 @@ int launch_dense_i4(TileArgs t, int nslots, hipStream_t st) {
 // dense down shares its 64 tokens' h16 across a block): mid loads run the wave gate/up (h out as h16) and the dense
 // down, on two pass lists.
 struct Plan {
-    bool tiled, dense_gu, dense_dn, mxd, wave_gu, wave_dn, mxw, h16, two_lists, ingroup;
+    bool tiled, dense_gu, dense_dn, mxd, wave_gu, wave_dn, mxw, h16, two_lists, ingroup, i4_ex;
     int nt, i4_m, P_gu, P_dn;
 };
 
@@ -1829,6 +1853,14 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
     const bool dense_gu_x = INT4 ? x_dtype != MOE_DTYPE_F32 : nx == 1;
     p.dense_gu = dense_gu_x && p.tiled && avg > min_avg &&
                  (dmode == 1 || (dmode < 0 && dblocks >= MOE_DENSE_MIN_BLOCKS));
+    // int4 up to the dense gate/up's line: the dense gate/up on exact weights (the wave tiles' codes are exact there, and the
+    // down's operands are fp16 already), 32-token passes at four blocks per CU, from 21 slots per expert. Layers, wave /
+    // exact dense: DeepSeek-V2-Lite T = 237 (29 slots) 141.4 / 128.3 us, Zipf 141.8 / 126.5; OLMoE T = 200 (25) 102.0 / 98.4,
+    // Zipf 109.5 / 101.8, T = 256 (32) 114.6 / 102.9; Mixtral T = 120 (30) 266 / 240; Qwen3-235B T = 300 (19) 370 / 347; but
+    // OLMoE T = 140 (18) 84.3 / 86.3, Qwen3 T = 300 (19) 120.9 / 121.5
+    p.i4_ex = INT4 && !p.dense_gu && dense_gu_x && p.tiled && avg > env_int("MOE_DENSE_EX_MIN_AVG", 20) && avg <= 32 &&
+              (dmode == 1 || (dmode < 0 && dblocks >= MOE_DENSE_MIN_BLOCKS));
+    p.dense_gu |= p.i4_ex;
     p.dense_dn = p.dense_gu || (INT4 && p.tiled && dmode != 0 && avg > dn_min_avg &&
                                 (dmode == 1 || dn_blocks >= MOE_DENSE_MIN_BLOCKS));
     p.mxd = mx_fit && p.dense_gu && w->F % 32 == 0 && w->d % 64 == 0;
@@ -1847,9 +1879,9 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
     // (64) 140 / 132, Qwen3 T = 544 (34, skew apart) 148.6 / 146.0, d = 1088 F = 704 T = 700 (53) 66.9 / 55.9, Mixtral
     // T = 512 (128) 486 / 484
     p.i4_m = avg <= 48 ? 16 : 32;
-    // pass lists: 16 nt tokens per pass for the wave tiles, 64 for the dense tiles; a second list when the two stages
+    // pass lists: 16 nt tokens per pass for the wave tiles, 64 for the dense tiles (32: exact weights); a second list when the two stages
     // take different kernels
-    p.P_gu = p.dense_gu ? DP : 16 * p.nt;
+    p.P_gu = p.i4_ex ? 32 : p.dense_gu ? DP : 16 * p.nt;
     p.P_dn = p.dense_dn ? DP : 16 * p.nt;
     p.two_lists = p.P_gu != p.P_dn;
     // both stages on the wave tiles with few slots: each workgroup can find its pass from the raw ids itself (an LDS
@@ -1936,12 +1968,14 @@ int run_tiles_fmt(const ExpertsArgs& a) {
             if (!rc) rc = launch_mxd<2, 2, 2>(g, nslots, a.st);
             if (rc) return rc;
         } else if (dense_gu && INT4) {
-            if (a.x_dtype == MOE_DTYPE_F16) k_x16<MOE_DTYPE_F16><<<a.T, 256, 0, a.st>>>(a.x, a.x16, a.xexp, w->d);
-            else k_x16<MOE_DTYPE_BF16><<<a.T, 256, 0, a.st>>>(a.x, a.x16, a.xexp, w->d);
+            uint8_t* xsum = pl.i4_ex ? a.xsum : nullptr;
+            if (a.x_dtype == MOE_DTYPE_F16) k_x16<MOE_DTYPE_F16><<<a.T, 256, 0, a.st>>>(a.x, a.x16, a.xexp, xsum, w->d);
+            else k_x16<MOE_DTYPE_BF16><<<a.T, 256, 0, a.st>>>(a.x, a.x16, a.xexp, xsum, w->d);
             rc = hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
             if (rc) return rc;
             g.actv = a.x16;
             g.xexp = a.xexp;
+            g.xsum = xsum;
         }
         if (mxw) {
             if (!a.xterm_ready) rc = launch_mx_terms<2>(a.xb, a.T, w->d, a.xterm, a.st);
@@ -1950,8 +1984,9 @@ int run_tiles_fmt(const ExpertsArgs& a) {
         } else if (mxd) rc = 0;
         else if (dense_gu) {
             if constexpr (!INT4) rc = launch_dense<2>(g, nslots, a.st);
-            else if (pl.i4_m == 16) rc = launch_dense_i4<2, 1, 16, 2>(g, nslots, a.st);
-            else rc = launch_dense_i4<2, 1, 32, 3>(g, nslots, a.st);
+            else if (pl.i4_ex) rc = launch_dense_i4<2, 1, 32, 32, 4, true>(g, nslots, a.st);
+            else if (pl.i4_m == 16) rc = launch_dense_i4<2, 1, 16, 64, 2>(g, nslots, a.st);
+            else rc = launch_dense_i4<2, 1, 32, 64, 3>(g, nslots, a.st);
         }
         else if (wave_gu && h16)
             rc = launch_wave_tile<FMT, 2, MOE_WAVE_RT_GU, MOE_WAVE_D_GU, INT4>(g, nt, nslots, a.st, a.nx);
@@ -2004,7 +2039,7 @@ int run_tiles_fmt(const ExpertsArgs& a) {
         } else if (dense_dn) {
             // int4: 32 rows per wave at four blocks per CU; 64 rows (three blocks) or 32-token tiles measured slower on
             // every shape but Qwen3 T = 4096 (even)
-            if constexpr (INT4) rc = launch_dense_i4<1, 1, 16, 4>(d, nslots, a.st);
+            if constexpr (INT4) rc = launch_dense_i4<1, 1, 16, 64, 4>(d, nslots, a.st);
             else rc = launch_dense<1>(d, nslots, a.st);
         }
         else if (wave_dn && wide_dn(MOE_WAVE_RT_DN_WIDE))

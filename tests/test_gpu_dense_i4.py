@@ -78,3 +78,43 @@ def test_slot_exponents_brought_together(monkeypatch, F):
     assert (y[7] == 0).all()
     for rows in (slice(0, None, 5), slice(1, None, 5), slice(3, None, 5)):
         assert_close(y[rows], want[rows], tol=5e-3, what=(F, rows))
+
+
+@pytest.mark.parametrize("d,F,dtype", [(128, 64, torch.bfloat16), (192, 320, torch.float16), (1088, 192, torch.bfloat16),
+                                       (64, 128, torch.bfloat16), (2048, 64, torch.float16)])
+@pytest.mark.parametrize("counts", [[32, 31, 33, 1, 24, 40, 16, 21], [64, 65, 0, 1, 0, 33, 31, 2]])
+def test_exact_weight_gate_up(monkeypatch, counts, d, F, dtype):
+    """21 to 32 slots per expert: the dense gate/up on exact weights, whose group biases go in as a product of their own.
+    Biases of every size (a wrong group-sum term is an O(1) error), inputs and scales spread over powers of two, against
+    the oracle and against the wave tiles' exact codes: both round h to the same fp16, so they differ by the h16 values on
+    which 1e-6 of h decides the rounding (a few in ten thousand, 2^-11 each): far below rounding weights to fp16 (2e-4)."""
+    from moelab_amd import _lib, experts, formats
+    monkeypatch.setenv("MOE_DENSE", "1")
+    E, T = len(counts), sum(counts)
+    assert 20 < (T + E - 1) // E <= 32
+    g = torch.Generator(device=DEV).manual_seed(T + d)
+
+    def proj(N, K):
+        codes, scales, _ = formats.random_int4(E, N, K, generator=g, device=DEV)
+        scales = (scales.float() * torch.exp2(torch.randint(-3, 4, scales.shape, generator=g, device=DEV).float())).to(torch.bfloat16)
+        return codes, scales, (torch.randn(scales.shape, generator=g, device=DEV) * 0.1).to(torch.bfloat16)
+    s = experts.make_state("int4", proj(F, d), proj(F, d), proj(d, F))
+    x = torch.randn((T, d), generator=g, device=DEV) * torch.exp2(torch.randint(-6, 7, (T, 1), generator=g, device=DEV).float())
+    x[3] = 0
+    x = x.to(dtype)
+    rng = np.random.default_rng(T)
+    idx = torch.from_numpy(rng.permutation(np.repeat(np.arange(E, dtype=np.int32), counts))[:, None].copy()).to(DEV)
+    wts = torch.ones((T, 1), device=DEV)
+    print(f"case exact gate/up d={d} F={F} {dtype} {counts}", flush=True)
+    got = {}
+    for least in ("20", "100"):
+        monkeypatch.setenv("MOE_DENSE_EX_MIN_AVG", least)
+        got[least] = experts.run_experts(s, x, idx, wts, path=_lib.PATH_GROUPED, out_dtype=torch.float32).double()
+    # In norms, row by row too: the rows' sizes span 2^24 (h grows with x^2) and single outputs have a heavy tail where few
+    # terms dominate. h and W_down each carry fp16's rounding, at most 2^-12 per term: sqrt(2) 2^-12 = 3.5e-4 of the norm
+    # (rows of few terms: four times that); the wave tiles' result carries the same.
+    want = torch.from_numpy(oracle_y(s, x, idx, wts)).to(DEV).double()
+    off, off_wave = ((got[k] - want).norm() / want.norm() for k in ("20", "100"))
+    assert off < 5e-4 and off < 1.25 * off_wave + 1e-6
+    assert ((got["20"] - want).norm(dim=1) <= 1.5e-3 * want.norm(dim=1)).all()
+    assert float((got["20"] - got["100"]).norm() / got["100"].norm()) < 5e-5
