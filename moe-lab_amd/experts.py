@@ -72,8 +72,9 @@ def unpack(s, n):
 
 def _desc(s):
     """ctypes moe_experts_t for a state (cached; rebuilt if any tensor changed)."""
-    tensors = (s["g"], s["u"], s["d"]) + tuple(s.get(b) for b in ("bg", "bu", "bd", "gt", "ut", "dt"))
-    key = tuple(0 if t is None else t.data_ptr() for t in tensors)
+    get = s.get
+    key = [0 if t is None else t.data_ptr() for t in (s["g"], s["u"], s["d"], get("bg"), get("bu"), get("bd"), get("gt"),
+                                                      get("ut"), get("dt"))]
     c = s.get("_c")
     if c is not None and c[0] == key:
         return c[1]
@@ -114,9 +115,9 @@ def run_experts(s, x, idx, wts, act=0, path=_lib.PATH_AUTO, nored=False, residua
         raise TypeError(f"activation dtype {x.dtype}: the expert kernels take bf16, fp16 or fp32")
     T, d = x.shape
     k = idx.shape[1]
-    x = x.contiguous()
-    idx = idx.to(torch.int32).contiguous()
-    wts = wts.to(torch.float32).contiguous()
+    x = _lib.dense(x)
+    idx = _lib.dense(idx, torch.int32)
+    wts = _lib.dense(wts, torch.float32)
     desc = _desc(s)
     L = _lib.lib()
     nbytes = L.moe_experts_workspace_bytes(desc, T, k, path)
@@ -125,7 +126,7 @@ def run_experts(s, x, idx, wts, act=0, path=_lib.PATH_AUTO, nored=False, residua
     if out is None:
         out = torch.empty((T * k if nored else T, d), dtype=out_dtype, device=x.device)
     assert out.dtype == out_dtype and out.dtype in _lib.DTYPE
-    res = None if residual is None else residual.to(out_dtype).contiguous()
+    res = None if residual is None else _lib.dense(residual, out_dtype)
     rc = L.moe_experts_run_stages(desc, _lib.ptr(x), _lib.DTYPE[x.dtype], _lib.ptr(idx), _lib.ptr(wts), T, k,
                                   int(act), int(path), int(bool(nored)), _lib.ptr(out), _lib.DTYPE[out.dtype],
                                   _lib.ptr(res), _lib.ptr(ws), ws.numel(), int(stages), _lib.stream_of(x.device))
@@ -166,9 +167,9 @@ def run_routed(s, x, wr, k, bias=None, norm=True, scale=1.0, act=0, residual=Non
     if x.dtype != torch.bfloat16 or wr.dtype != torch.bfloat16:
         raise TypeError("run_routed takes bf16 x and router weights (the gate GEMV reads bf16)")
     T, d = x.shape
-    x = x.contiguous()
-    wr = wr.contiguous()
-    b = None if bias is None else bias.to(torch.float32).contiguous()
+    x = _lib.dense(x)
+    wr = _lib.dense(wr)
+    b = None if bias is None else _lib.dense(bias, torch.float32)
     desc = _desc(s)
     L = _lib.lib()
     S = int(s.get("n_shared", 0))
@@ -183,10 +184,10 @@ def run_routed(s, x, wr, k, bias=None, norm=True, scale=1.0, act=0, residual=Non
     assert out.dtype == out_dtype and out.dtype in _lib.DTYPE
     idx = torch.empty((T, k), dtype=torch.int32, device=x.device)
     wts = torch.empty((T, k), dtype=torch.float32, device=x.device)
-    res = None if residual is None else residual.to(out_dtype).contiguous()
+    res = None if residual is None else _lib.dense(residual, out_dtype)
     if S:
         g = s.get("shared_gate")
-        g = None if g is None else g.to(torch.bfloat16).contiguous()
+        g = None if g is None else _lib.dense(g, torch.bfloat16)
         rc = L.moe_layer_run_shared(desc, S, _lib.ptr(x), _lib.DTYPE[x.dtype], _lib.ptr(wr), _lib.ptr(b), _lib.ptr(g),
                                     T, k, int(bool(norm)), float(scale), int(act), _lib.ptr(idx), _lib.ptr(wts),
                                     _lib.ptr(out), _lib.DTYPE[out.dtype], _lib.ptr(res), _lib.ptr(ws), ws.numel(),
@@ -211,7 +212,7 @@ def run_shared(s, x, gate=None, act=0, residual=None, out=None, out_dtype=None):
     if x.dtype not in _lib.DTYPE:
         raise TypeError(f"activation dtype {x.dtype}: the expert kernels take bf16, fp16 or fp32")
     T, d = x.shape
-    x = x.contiguous()
+    x = _lib.dense(x)
     desc = _desc(s)
     L = _lib.lib()
     ws = _lib.workspace(x.device, L.moe_shared_experts_workspace_bytes(desc, T))
@@ -219,8 +220,8 @@ def run_shared(s, x, gate=None, act=0, residual=None, out=None, out_dtype=None):
     if out is None:
         out = torch.empty((T, d), dtype=out_dtype, device=x.device)
     assert out.dtype == out_dtype and out.dtype in _lib.DTYPE
-    res = None if residual is None else residual.to(out_dtype).contiguous()
-    g = None if gate is None else gate.to(torch.bfloat16).contiguous()
+    res = None if residual is None else _lib.dense(residual, out_dtype)
+    g = None if gate is None else _lib.dense(gate, torch.bfloat16)
     rc = L.moe_shared_experts_run(desc, _lib.ptr(x), _lib.DTYPE[x.dtype], T, int(act), _lib.ptr(g), _lib.ptr(out),
                                   _lib.DTYPE[out.dtype], _lib.ptr(res), _lib.ptr(ws), ws.numel(),
                                   _lib.stream_of(x.device))
@@ -267,9 +268,9 @@ def run_experts_shared(s, x, idx, wts, act=0, path=_lib.PATH_AUTO, residual=None
     T, d = x.shape
     k = int(idx.shape[1])
     S = int(s["n_shared"])
-    x = x.contiguous()
-    idx = idx.to(torch.int32).contiguous()
-    wts = wts.to(torch.float32).contiguous()
+    x = _lib.dense(x)
+    idx = _lib.dense(idx, torch.int32)
+    wts = _lib.dense(wts, torch.float32)
     desc = _desc(s)
     L = _lib.lib()
     ws = _lib.workspace(x.device, L.moe_experts_shared_workspace_bytes(desc, S, T, k, int(path)))
@@ -277,9 +278,9 @@ def run_experts_shared(s, x, idx, wts, act=0, path=_lib.PATH_AUTO, residual=None
     if out is None:
         out = torch.empty((T, d), dtype=out_dtype, device=x.device)
     assert out.dtype == out_dtype and out.dtype in _lib.DTYPE
-    res = None if residual is None else residual.to(out_dtype).contiguous()
+    res = None if residual is None else _lib.dense(residual, out_dtype)
     g = s.get("shared_gate")
-    g = None if g is None else g.to(torch.bfloat16).contiguous()
+    g = None if g is None else _lib.dense(g, torch.bfloat16)
     rc = L.moe_experts_run_shared(desc, S, _lib.ptr(x), _lib.DTYPE[x.dtype], _lib.ptr(idx), _lib.ptr(wts), T, k,
                                   int(act), int(path), _lib.ptr(g), _lib.ptr(out), _lib.DTYPE[out.dtype],
                                   _lib.ptr(res), _lib.ptr(ws), ws.numel(), _lib.stream_of(x.device))
