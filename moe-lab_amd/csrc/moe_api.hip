@@ -268,7 +268,7 @@ namespace {
 int experts_call(const moe_experts_t* w, const void* x, int x_dtype, const int32_t* idx, const float* wts, int T, int k,
                  int act, int path, int nored, void* y, int y_dtype, const void* residual, void* workspace,
                  size_t workspace_bytes, int stages, void* stream, const float* route_logits, int route_norm,
-                 float route_scale, int pregrouped = 0, int xterm_ready = 0);
+                 float route_scale, int pregrouped = 0, int x_ready = 0);
 int layer_call(const moe_experts_t* w, int S, const void* x, int x_dtype, const void* wr, const float* wr_bias,
                const void* gate, int T, int k, int norm, float scale, int act, int32_t* idx, float* wts, void* y,
                int y_dtype, const void* residual, void* workspace, size_t workspace_bytes, void* stream);
@@ -315,7 +315,7 @@ namespace {
 int experts_call(const moe_experts_t* w, const void* x, int x_dtype, const int32_t* idx, const float* wts, int T, int k,
                  int act, int path, int nored, void* y, int y_dtype, const void* residual, void* workspace,
                  size_t workspace_bytes, int stages, void* stream, const float* route_logits, int route_norm,
-                 float route_scale, int pregrouped, int xterm_ready) {
+                 float route_scale, int pregrouped, int x_ready) {
     if (stages < 1 || stages > MOE_STAGE_ALL) return MOE_ERR_ARG;
     int rc = check_experts(w);
     if (rc) return rc;
@@ -380,7 +380,8 @@ int experts_call(const moe_experts_t* w, const void* x, int x_dtype, const int32
         a.grp.chunks = (int32_t*)(ws + L.yp);   // the down's output space, free until the down runs
         a.grp.chunks_n = (size_t)T * k * w->d;
         a.pregrouped = pregrouped;
-        a.xterm_ready = a.xterm ? xterm_ready : 0;
+        a.xterm_ready = a.xterm ? x_ready : 0;   // the router wrote x in the form the gate/up reads: terms or x16
+        a.x16_ready = x_ready;
     }
     return rpath == MOE_PATH_GROUPED ? moe::run_experts_tiles(a) : moe::run_experts_slots(a);
 }
@@ -434,12 +435,15 @@ int layer_call(const moe_experts_t* w, int S, const void* x, int x_dtype, const 
         return experts_call(w, x, x_dtype, idx, wts, T, k, act, MOE_PATH_AUTO, 0, y, y_dtype, residual, workspace,
                             L.total, MOE_STAGE_ALL, stream, ra.logits, norm, scale);
     }
-    int pregrouped = 0, xterm_ready = 0;
+    int pregrouped = 0, x_ready = 0;
     if (resolve_path(MOE_PATH_AUTO, T) == MOE_PATH_GROUPED) {
         const moe::TilePasses tp = moe::tile_passes(w, T, ks, x_dtype);
         if (tp.mx) {   // the block-scaled MXFP4 tiles: the finishing launch also writes x's term records
             ra.xterm = (uint8_t*)(ws + L.xp);
-            xterm_ready = 1;
+            x_ready = 1;
+        } else if (tp.x16) {   // the int4 dense gate/up: its fp16 rows (4-5 us less than a launch of their own at T = 237, 512)
+            ra.x16 = moe::X16Out{(uint16_t*)(ws + L.x16), (int32_t*)(ws + L.xexp), tp.ex ? (uint8_t*)(ws + L.xp) : nullptr};
+            x_ready = 1;
         }
         if (!(tp.ingroup && moe::env_int("MOE_LAYER_INGROUP", 1))) {
             ra.grp = moe::GroupBufs{(int32_t*)(ws + L.counts), (int32_t*)(ws + L.offsets), (int32_t*)(ws + L.sorted),
@@ -453,7 +457,7 @@ int layer_call(const moe_experts_t* w, int S, const void* x, int x_dtype, const 
     rc = moe::launch_route(ra, true, st);
     if (rc) return rc;
     return experts_call(w, x, x_dtype, eidx, ewts, T, ks, act, MOE_PATH_AUTO, 0, y, y_dtype, residual, workspace,
-                        L.total, MOE_STAGE_ALL, stream, nullptr, 1, 1.f, pregrouped, xterm_ready);
+                        L.total, MOE_STAGE_ALL, stream, nullptr, 1, 1.f, pregrouped, x_ready);
 }
 
 }  // namespace

@@ -21,6 +21,13 @@ struct GroupBufs {
     size_t chunks_n;  // its room in ints
 };
 
+// x16 of the int4 dense gate/up (moe_x16.h)
+struct X16Out {
+    uint16_t* x16;   // [T, d] fp16, or null: not written
+    int32_t* xexp;   // [T]
+    uint8_t* xsum;   // group sums for the exact-weight gate/up, or null
+};
+
 // One router launch (moe_router.hip): the logits, then (tail) the top-k tail per token, the merged slot lists with
 // shared experts, and the slot grouping.
 // Field order: the logits launch's prologue reads the first 64-byte scalar-cache line only; the tail launch's
@@ -45,6 +52,7 @@ struct RouterArgs {
     int P;                 // pass size of grp.items (unused when null)
     GroupBufs grp;         // grp.counts null: no grouping; else the grouping of the slots (sidx when S > 0, else idx)
     int P2;                // pass size of grp.items2
+    X16Out x16;            // x16.x16 or null: the tails' launch also writes x's fp16 rows (the int4 dense gate/up's, as k_x16)
     uint8_t* xterm;        // or null: route_finish also writes x's 2-term fp8 records here (the block-scaled MXFP4
                            // tiles' activations, as k_mx_terms would), so the experts call launches no k_mx_terms
 };
@@ -78,6 +86,7 @@ struct TilePasses {
     int P, P2, ingroup;
     int mx;   // the call runs the block-scaled MXFP4 tiles, which read x as 2-term fp8 records (xterm)
     int x16;  // the call's gate/up reads x as x16 (k_x16), not as bf16 planes
+    int ex;   // on exact weights: x16 comes with its group sums
 };
 TilePasses tile_passes(const moe_experts_t* w, int T, int k, int x_dtype);
 
@@ -103,6 +112,7 @@ struct ExpertsArgs {
     uint8_t* xterm; // grouped path, MXFP4 block-scaled MFMA: x's fp8 term records (the x-planes region when x is bf16)
     GroupBufs grp;  // grouped path
     int pregrouped; // grouped path: grp already holds the grouping and pass lists of idx (written by the router)
+    int x16_ready;   // grouped path: x16, xexp (and xsum) already hold x's rows (written by the router)
     int xterm_ready; // grouped path: xterm already holds x's term records (written by the router)
     int stages;     // bit 0: grouping + gate/up (writes h), bit 1: down + combine (reads h)
     // moe_layer_run at T == 1: the gate/up waves take their experts from the top-k of these router logits [T, E] (and

@@ -21,6 +21,7 @@
 #include "moe_group.h"
 #include "moe_internal.h"
 #include "moe_mxterms.h"
+#include "moe_x16.h"
 
 namespace moe {
 
@@ -254,6 +255,10 @@ __global__ void __launch_bounds__(64 * FIN_WAVES) route_finish(RouterArgs a) {
             else ids[(size_t)t * ws + lane] = sid;
         }
     }
+    if (a.x16.x16 && wave >= FIN_TOK && wave < 2 * FIN_TOK) {   // x's fp16 rows, one wave per token beside the tails
+        const int tx = blockIdx.x * FIN_TOK + wave - FIN_TOK;
+        if (tx < a.T) x16_row<MOE_DTYPE_BF16>(a.x, tx, a.x16, a.d);
+    }
     if (a.xterm) {
         // x's 2-term fp8 records for the block-scaled MXFP4 tiles (what k_mx_terms writes), for this workgroup's
         // tokens: one thread per 32-input block, numbered from wave FIN_TOK on, so that the waves that ran the
@@ -316,6 +321,7 @@ __global__ void __launch_bounds__(64 * SPLIT_WAVES) route_tails(RouterArgs a, in
             ids[(size_t)t * ws + lane] = sid;
             atomicAdd(&sm[sid], 1);
         }
+        if (a.x16.x16) x16_row<MOE_DTYPE_BF16>(a.x, t, a.x16, a.d);
     }
     if (a.xterm) {   // x's fp8 term records, as in route_finish
         const int nsl = (a.d + 127) >> 7;

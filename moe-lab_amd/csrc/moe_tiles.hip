@@ -29,6 +29,7 @@
 #include "moe_group.h"
 #include "moe_internal.h"
 #include "moe_mxterms.h"
+#include "moe_x16.h"
 
 #include <math.h>
 #include <stdlib.h>
@@ -41,21 +42,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2x __attribute__((ext_vector_type(2)));
 
-// Power-of-two exponent e with which the int4 dense tiles store a row (x16: a token's x; h16: a slot's 32-row chunk
-// of h) of largest magnitude amax as fp16 v 2^-e: 0 while 2^-8 <= amax < 2^15 (fp16's subnormal rounding, 2^-25,
-// then stays below 2^-17 of the row's largest), else floor(log2 amax) - 14, which puts the largest at [2^14, 2^15)
-// (large rows: no overflow; small rows: no flush to zero), clamped to [-127, 127]. An all-zero row gives
-// H16_ZERO_EXP, which never wins a slot's maximum (its values are 0 under any scaling); NaN gives 0.
-constexpr int H16_ZERO_EXP = -128;
-__device__ __forceinline__ int h16_exponent(float amax) {
-    if (amax == 0.f) return H16_ZERO_EXP;
-    if (!(amax < 32768.f && amax >= 0.00390625f)) {
-        if (amax != amax) return 0;
-        const int e = (int)((__float_as_uint(amax) >> 23) & 0xFFu) - 141;
-        return e < -127 ? -127 : (e > 127 ? 127 : e);
-    }
-    return 0;
-}
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int TL_ROWS = 64;   // weight rows per block
@@ -1454,93 +1440,11 @@ int launch_mx_terms(const uint16_t* src, int rows, int K, uint8_t* out, hipStrea
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
-// Dense int4, before gate/up: x [T, d] (bf16 or fp16) -> x16 = x 2^-E fp16, one block per token, E = h16_exponent of
-// the row's largest |x| (bf16 and fp16 to fp16 are then exact except far below the row's largest, where fp16's
-// subnormal range rounds); E per token for the gate/up epilogue.
-// 8 activations of x (bf16, fp16 or fp32) starting at element 8c of row `row`, as fp32
+// Dense int4, before gate/up, where the router has not written it already: one wave per token (x16_row)
 template <int XDT>
-__device__ __forceinline__ void load_x8(const void* row, int c, float v[8]) {
-    if (XDT == MOE_DTYPE_F32) {
-        const float4 a = reinterpret_cast<const float4*>(row)[2 * c], b = reinterpret_cast<const float4*>(row)[2 * c + 1];
-        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-        return;
-    }
-    const uint4 r = reinterpret_cast<const uint4*>(row)[c];
-    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if (XDT == MOE_DTYPE_F16) {
-            v[2 * q] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[q] & 0xFFFFu));
-            v[2 * q + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[q] >> 16));
-        } else {
-            v[2 * q] = bf16lo(w[q]);
-            v[2 * q + 1] = bf16hi(w[q]);
-        }
-    }
-}
-
-// xsum (the exact-weight gate/up): also the sums of x16 over the 64-input groups, 16 bytes per token and 128-input slice in
-// A-operand form: XS 2^-6 of its two groups as fp16 hi + lo, (hi0, hi1, hi0, hi1, lo0, lo1, 0, 0). x16 then takes the
-// exponent that puts every row's largest at [2^14, 2^15), so that bf16 rows keep inputs down to 2^-38 of it.
-template <int XDT>
-__global__ void __launch_bounds__(256) k_x16(const void* __restrict__ x, uint16_t* __restrict__ x16,
-                                             int32_t* __restrict__ xexp, uint8_t* __restrict__ xsum, int d) {
-    __shared__ float sM[4];
-    const int t = blockIdx.x, tid = threadIdx.x;
-    const void* row = reinterpret_cast<const uint8_t*>(x) + (size_t)t * d * (XDT == MOE_DTYPE_F32 ? 4 : 2);
-    uint4* out = reinterpret_cast<uint4*>(x16 + (size_t)t * d);
-    const int nch = d >> 3;   // 8-element chunks; d <= 2048 * 8 for one round of 8 per thread
-    constexpr int CPT = 8;
-    float am = 0.f;
-    for (int c0 = 0; c0 < nch; c0 += 256 * CPT) {
-        float v[CPT][8];
-#pragma unroll
-        for (int i = 0; i < CPT; ++i)
-            if (c0 + i * 256 + tid < nch) load_x8<XDT>(row, c0 + i * 256 + tid, v[i]);
-#pragma unroll
-        for (int i = 0; i < CPT; ++i)
-            if (c0 + i * 256 + tid < nch) {
-#pragma unroll
-                for (int q = 0; q < 8; ++q) am = fmaxf(am, fabsf(v[i][q]));
-            }
-    }
-    for (int o = 32; o; o >>= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
-    if ((tid & 63) == 0) sM[tid >> 6] = am;
-    __syncthreads();
-    const float amax = fmaxf(fmaxf(sM[0], sM[1]), fmaxf(sM[2], sM[3]));
-    int E = h16_exponent(amax);
-    if (xsum && E == 0 && amax == amax) {   // an ordinary row: the same rule as for the large and small ones
-        E = (int)((__float_as_uint(amax) >> 23) & 0xFFu) - 141;
-    }
-    if (tid == 0) xexp[t] = E;
-    for (int c0 = 0; c0 < nch; c0 += 256) {   // the row again (cache hits)
-        const int c = c0 + tid;
-        float sum = 0.f;
-        if (c < nch) {
-            float v[8];
-            load_x8<XDT>(row, c, v);
-            uint32_t o4[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const _Float16 lo = (_Float16)__builtin_ldexpf(v[2 * q], -E), hi = (_Float16)__builtin_ldexpf(v[2 * q + 1], -E);
-                o4[q] = (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
-                sum += (float)lo + (float)hi;
-            }
-            out[c] = make_uint4(o4[0], o4[1], o4[2], o4[3]);
-        }
-        if (xsum) {   // 8 chunks per group, 16 per slice; a slice that ends at input 64 has a zero second group
-            sum = sum_lanes<8>(sum);
-            const float s1 = __shfl(sum, (tid & 63) | 8, 64);
-            if (c < nch && (c & 15) == 0) {
-                const float w0 = sum * 0x1p-6f, w1 = s1 * 0x1p-6f;
-                const _Float16 h0 = (_Float16)w0, h1 = (_Float16)w1;
-                const _Float16 l0 = (_Float16)(w0 - (float)h0), l1 = (_Float16)(w1 - (float)h1);
-                const uint32_t hh = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-                const uint32_t ll = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
-                reinterpret_cast<uint4*>(xsum)[(size_t)t * ((d + 127) >> 7) + (c >> 4)] = make_uint4(hh, hh, ll, 0u);
-            }
-        }
-    }
+__global__ void __launch_bounds__(256) k_x16(const void* __restrict__ x, int T, X16Out o, int d) {
+    const int t = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (t < T) x16_row<XDT>(x, t, o, d);
 }
 
 // int4 grouped path, between gate/up and a dense down. The gate/up wrote h16 = h 2^-e with e per (slot, 32-row chunk)
@@ -1969,10 +1873,13 @@ int run_tiles_fmt(const ExpertsArgs& a) {
             if (rc) return rc;
         } else if (dense_gu && INT4) {
             uint8_t* xsum = pl.i4_ex ? a.xsum : nullptr;
-            if (a.x_dtype == MOE_DTYPE_F16) k_x16<MOE_DTYPE_F16><<<a.T, 256, 0, a.st>>>(a.x, a.x16, a.xexp, xsum, w->d);
-            else k_x16<MOE_DTYPE_BF16><<<a.T, 256, 0, a.st>>>(a.x, a.x16, a.xexp, xsum, w->d);
-            rc = hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
-            if (rc) return rc;
+            if (!a.x16_ready) {
+                const X16Out o{a.x16, a.xexp, xsum};
+                if (a.x_dtype == MOE_DTYPE_F16) k_x16<MOE_DTYPE_F16><<<(a.T + 3) / 4, 256, 0, a.st>>>(a.x, a.T, o, w->d);
+                else k_x16<MOE_DTYPE_BF16><<<(a.T + 3) / 4, 256, 0, a.st>>>(a.x, a.T, o, w->d);
+                rc = hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
+                if (rc) return rc;
+            }
             g.actv = a.x16;
             g.xexp = a.xexp;
             g.xsum = xsum;
@@ -2064,7 +1971,7 @@ int run_experts_tiles(const ExpertsArgs& a) {
 TilePasses tile_passes(const moe_experts_t* w, int T, int k, int x_dtype) {
     const Plan p = w->fmt == MOE_FMT_INT4_G64 ? make_plan<FmtInt4>(w, T, k, x_dtype) : make_plan<FmtMxfp4>(w, T, k, x_dtype);
     return TilePasses{p.P_gu, p.two_lists ? p.P_dn : 0, p.ingroup ? 1 : 0, p.mxd || p.mxw ? 1 : 0,
-                      w->fmt == MOE_FMT_INT4_G64 && p.dense_gu ? 1 : 0};
+                      w->fmt == MOE_FMT_INT4_G64 && p.dense_gu ? 1 : 0, p.i4_ex ? 1 : 0};
 }
 
 int launch_pack_tiles(int fmt, int E, int N, int K, const void* rows, void* tiles, hipStream_t st) {

@@ -118,3 +118,21 @@ def test_exact_weight_gate_up(monkeypatch, counts, d, F, dtype):
     assert off < 5e-4 and off < 1.25 * off_wave + 1e-6
     assert ((got["20"] - want).norm(dim=1) <= 1.5e-3 * want.norm(dim=1)).all()
     assert float((got["20"] - got["100"]).norm() / got["100"].norm()) < 5e-5
+
+
+@pytest.mark.parametrize("T,E,k,d", [(150, 16, 3, 192), (61, 8, 4, 2112), (340, 16, 3, 128), (1100, 8, 2, 320)])
+def test_router_writes_the_fp16_rows(T, E, k, d, monkeypatch):
+    """A layer call whose router writes x16 (beside the tails of one-workgroup groupings, with the split tails otherwise;
+    with the group sums at 21 to 32 slots per expert) against routing first and calling the experts on the ids: the same
+    bits."""
+    from moelab_amd import experts, router
+    from moelab_amd.problem import baseline_int4_layer
+    from moelab_amd.shapes import MoEShape
+    monkeypatch.setenv("MOE_DENSE", "1")
+    s = baseline_int4_layer(MoEShape("t", d=d, f=128, E=E, k=k), seed=T, device=DEV)
+    wr = s.pop("wr")
+    x = (torch.randn((T, d), device=DEV) * torch.exp2(torch.randint(-12, 20, (T, 1), device=DEV).float())).to(torch.bfloat16)
+    y, idx, wts = experts.run_routed(s, x, wr, k, out_dtype=torch.float32)
+    i2, w2 = router.route(x, wr, k)
+    assert torch.equal(idx, i2) and torch.equal(wts, w2)
+    assert torch.equal(y, experts.run_experts(s, x, idx, wts, out_dtype=torch.float32))
