@@ -160,7 +160,7 @@ int moe_router_group(const void* x, const void* wr, const float* bias, int T, in
     moe::RouterArgs a{};
     a.x = (const uint16_t*)x, a.wr = (const uint16_t*)wr, a.bias = bias, a.T = T, a.d = d, a.E = E, a.k = k;
     a.norm = norm, a.scale = scale, a.logits = logits, a.lstride = E, a.idx = idx, a.wts = wts;
-    a.grp = moe::GroupBufs{counts, offsets, sorted, active, meta, nullptr, nullptr, nullptr, 0};
+    a.grp = moe::GroupBufs{counts, offsets, sorted, active, meta, nullptr, nullptr};
     return moe::launch_route(a, true, (hipStream_t)stream);
 }
 
@@ -176,8 +176,8 @@ int moe_group(const int32_t* idx, int n, int E, int32_t* counts, int32_t* offset
               int32_t* meta, void* stream) {
     if (n < 0 || E < 1 || E > 8192) return MOE_ERR_ARG;
     if (!counts || !offsets || !active || !meta || (n > 0 && (!idx || !sorted))) return MOE_ERR_ARG;
-    const moe::GroupBufs o{counts, offsets, sorted, active, meta, nullptr, nullptr, nullptr, 0};
-    return moe::launch_group(idx, n, E, o, (hipStream_t)stream);
+    const moe::GroupBufs o{counts, offsets, sorted, active, meta, nullptr, nullptr};
+    return moe::launch_group(idx, n, E, o, moe::GroupScratch{}, (hipStream_t)stream);
 }
 
 size_t moe_experts_workspace_bytes(const moe_experts_t* w, int T, int k, int path) {
@@ -377,8 +377,7 @@ int experts_call(const moe_experts_t* w, const void* x, int x_dtype, const int32
         a.grp.meta = (int32_t*)(ws + L.meta);
         a.grp.items = (int32_t*)(ws + L.items);
         a.grp.items2 = (int32_t*)(ws + L.items2);
-        a.grp.chunks = (int32_t*)(ws + L.yp);   // the down's output space, free until the down runs
-        a.grp.chunks_n = (size_t)T * k * w->d;
+        a.gsc = moe::GroupScratch{(int32_t*)(ws + L.yp), (size_t)T * k * w->d};   // the down's output space, free until then
         a.pregrouped = pregrouped;
         a.xterm_ready = a.xterm ? x_ready : 0;   // the router wrote x in the form the gate/up reads: terms or x16
         a.x16_ready = x_ready;
@@ -448,8 +447,8 @@ int layer_call(const moe_experts_t* w, int S, const void* x, int x_dtype, const 
         if (!(tp.ingroup && moe::env_int("MOE_LAYER_INGROUP", 1))) {
             ra.grp = moe::GroupBufs{(int32_t*)(ws + L.counts), (int32_t*)(ws + L.offsets), (int32_t*)(ws + L.sorted),
                                     (int32_t*)(ws + L.active), (int32_t*)(ws + L.meta), (int32_t*)(ws + L.items),
-                                    tp.P2 ? (int32_t*)(ws + L.items2) : nullptr, (int32_t*)(ws + L.yp),
-                                    (size_t)T * ks * w->d};
+                                    tp.P2 ? (int32_t*)(ws + L.items2) : nullptr};
+            ra.gsc = moe::GroupScratch{(int32_t*)(ws + L.yp), (size_t)T * ks * w->d};
             ra.P = tp.P, ra.P2 = tp.P2;
             pregrouped = 1;
         }

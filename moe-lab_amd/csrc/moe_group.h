@@ -222,7 +222,8 @@ __host__ __device__ inline int group_place_lds_ints(int E) { return (GROUP_PW + 
 // counts, offsets, the active list, the pass lists and meta (as group_block) and places none. sm:
 // group_place_lds_ints(E) ints.
 __device__ __forceinline__ void group_place(const int32_t* __restrict__ ids, int n, int E, int cs, int nchunk,
-                                            const GroupBufs& o, int P, int P2, int32_t* sm) {
+                                            const int32_t* __restrict__ chunks, const GroupBufs& o, int P, int P2,
+                                            int32_t* sm) {
     const int NT = (int)blockDim.x, NW = NT >> 6;
     int32_t* cur = sm;                      // [GROUP_PW][E]: the placing waves' counts, then their cursors
     int32_t* base = sm + GROUP_PW * E;      // slots of the earlier chunks
@@ -244,7 +245,7 @@ __device__ __forceinline__ void group_place(const int32_t* __restrict__ ids, int
             for (int r = s; r < nchunk; r += U * ns) {
                 int v[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) v[u] = r + u * ns < nchunk ? o.chunks[(size_t)(r + u * ns) * E + e] : 0;
+                for (int u = 0; u < U; ++u) v[u] = r + u * ns < nchunk ? chunks[(size_t)(r + u * ns) * E + e] : 0;
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     sa += v[u];

@@ -17,8 +17,11 @@ struct GroupBufs {
     int32_t* meta;    // [4]: active experts, bad ids, passes of the work list, passes of the second list
     int32_t* items;   // pass list, room for max_passes(n, E, 16) (expert, pass, passes) triples
     int32_t* items2;  // second pass list (dense down after wave gate/up), room for max_passes(n, E, 64)
-    int32_t* chunks;  // scratch of the two-launch grouping (per-chunk counts), or null: one workgroup groups the slots
-    size_t chunks_n;  // its room in ints
+};
+// scratch of the two-launch grouping (per-chunk counts; n: its room in ints), or null: one workgroup groups the slots
+struct GroupScratch {
+    int32_t* chunks;
+    size_t n;
 };
 
 // x16 of the int4 dense gate/up (moe_x16.h)
@@ -52,6 +55,7 @@ struct RouterArgs {
     int P;                 // pass size of grp.items (unused when null)
     GroupBufs grp;         // grp.counts null: no grouping; else the grouping of the slots (sidx when S > 0, else idx)
     int P2;                // pass size of grp.items2
+    GroupScratch gsc;
     X16Out x16;            // x16.x16 or null: the tails' launch also writes x's fp16 rows (the int4 dense gate/up's, as k_x16)
     uint8_t* xterm;        // or null: route_finish also writes x's 2-term fp8 records here (the block-scaled MXFP4
                            // tiles' activations, as k_mx_terms would), so the experts call launches no k_mx_terms
@@ -68,8 +72,9 @@ int launch_router_logits(const uint16_t* x, const uint16_t* wr, const float* bia
 int launch_topk(const void* logits, int dtype, int T, int E, int k, int norm, float scale, int32_t* idx, float* wts,
                 hipStream_t st, int lstride = 0);
 // stable grouping of the ids idx[n] into o (with o.items / o.items2 also the grouped kernels' pass lists, passes of P and
-// P2 slots); with o.chunks and many slots in two launches, else in one workgroup
-int launch_group(const int32_t* idx, int n, int E, const GroupBufs& o, hipStream_t st, int P = 0, int P2 = 0);
+// P2 slots); with sc.chunks and many slots in two launches, else in one workgroup
+int launch_group(const int32_t* idx, int n, int E, const GroupBufs& o, const GroupScratch& sc, hipStream_t st, int P = 0,
+                 int P2 = 0);
 // tuning and test knobs from the environment, read per call
 inline int env_int(const char* name, int dflt) {
     const char* v = getenv(name);
@@ -111,6 +116,7 @@ struct ExpertsArgs {
     uint8_t* xsum;  // grouped path, dense int4 on exact weights: x16's group sums (the x-planes region: x16 is read instead)
     uint8_t* xterm; // grouped path, MXFP4 block-scaled MFMA: x's fp8 term records (the x-planes region when x is bf16)
     GroupBufs grp;  // grouped path
+    GroupScratch gsc;
     int pregrouped; // grouped path: grp already holds the grouping and pass lists of idx (written by the router)
     int x16_ready;   // grouped path: x16, xexp (and xsum) already hold x's rows (written by the router)
     int xterm_ready; // grouped path: xterm already holds x's term records (written by the router)

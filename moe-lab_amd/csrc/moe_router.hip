@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(64 * FIN_WAVES) route_finish(RouterArgs a) {
 }
 
 // The same for calls with many slots (two-launch grouping, moe_group.h): SPLIT_WAVES tokens at a time, one per wave,
-// tok tokens per workgroup (a chunk), whose slots are counted per expert in LDS and written to a.grp.chunks[workgroup].
+// tok tokens per workgroup (a chunk), whose slots are counted per expert in LDS and written to a.gsc.chunks[workgroup].
 // Every SIMD runs four tails at once here (they are VALU-issue bound), where route_finish spreads few tails over many
 // CUs.
 constexpr int SPLIT_WAVES = 16;
@@ -329,7 +329,7 @@ __global__ void __launch_bounds__(64 * SPLIT_WAVES) route_tails(RouterArgs a, in
             mx_terms_block<2>(a.x + (size_t)t0 * a.d, t1 - t0, a.d, a.xterm + (size_t)t0 * nsl * mx_rec<2>(), i);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < Eg; i += 64 * SPLIT_WAVES) a.grp.chunks[(size_t)blockIdx.x * Eg + i] = sm[i];
+    for (int i = threadIdx.x; i < Eg; i += 64 * SPLIT_WAVES) a.gsc.chunks[(size_t)blockIdx.x * Eg + i] = sm[i];
 }
 
 // Two-launch grouping of given ids: the counts of each chunk of cs slots, then the placing workgroups.
@@ -347,9 +347,9 @@ __global__ void __launch_bounds__(256) k_group_count(const int32_t* __restrict__
     for (int i = threadIdx.x; i < E; i += 256) chunks[(size_t)blockIdx.x * E + i] = sm[i];
 }
 __global__ void __launch_bounds__(1024) k_group_place(const int32_t* __restrict__ idx, int n, int E, int cs, int nchunk,
-                                                      GroupBufs o, int P, int P2) {
+                                                      const int32_t* __restrict__ chunks, GroupBufs o, int P, int P2) {
     extern __shared__ int32_t sm[];
-    group_place(idx, n, E, cs, nchunk, o, P, P2, sm);
+    group_place(idx, n, E, cs, nchunk, chunks, o, P, P2, sm);
 }
 
 // Router tail on given logits [T, E] (fp32, bf16 or fp16): one wave per token.
@@ -431,13 +431,13 @@ shared_route(const void* __restrict__ x, int xdt, const uint16_t* __restrict__ g
 constexpr size_t FIN_LDS = 32 * 1024;
 
 // whether a call's grouping is split over chunks (two launches): enough slots, and scratch for the count rows
-static bool group_split(int n, int E, int nchunk, const GroupBufs& o) {
-    return o.chunks && n >= env_int("MOE_GROUP_SPLIT_MIN", GROUP_SPLIT_MIN) && E <= GROUP_SPLIT_MAX_E &&
-           (size_t)nchunk * E <= o.chunks_n;
+static bool group_split(int n, int E, int nchunk, const GroupScratch& sc) {
+    return sc.chunks && n >= env_int("MOE_GROUP_SPLIT_MIN", GROUP_SPLIT_MIN) && E <= GROUP_SPLIT_MAX_E &&
+           (size_t)nchunk * E <= sc.n;
 }
-static int launch_group_place(const int32_t* idx, int n, int E, int cs, int nchunk, const GroupBufs& o, int P, int P2,
-                              hipStream_t st) {
-    k_group_place<<<nchunk + 1, 1024, (size_t)group_place_lds_ints(E) * 4, st>>>(idx, n, E, cs, nchunk, o, P, P2);
+static int launch_group_place(const int32_t* idx, int n, int E, int cs, int nchunk, const int32_t* chunks,
+                              const GroupBufs& o, int P, int P2, hipStream_t st) {
+    k_group_place<<<nchunk + 1, 1024, (size_t)group_place_lds_ints(E) * 4, st>>>(idx, n, E, cs, nchunk, chunks, o, P, P2);
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
@@ -466,7 +466,7 @@ int launch_route(RouterArgs a, bool tail, hipStream_t st) {
         return MOE_ERR_ARG;   // pass sizes are powers of two
     const int n_all = a.T * (a.k + a.S), E_all = a.E + a.S;
     const int tok = group_chunk(a.T, SPLIT_WAVES), nchunk = (a.T + tok - 1) / tok;
-    const bool split = tail && a.grp.counts && group_split(n_all, E_all, nchunk, a.grp);
+    const bool split = tail && a.grp.counts && group_split(n_all, E_all, nchunk, a.gsc);
     if (split) a.arrive = nullptr;
     int rc = launch_route_logits(a, st);
     if (rc || !tail) return rc;
@@ -477,7 +477,7 @@ int launch_route(RouterArgs a, bool tail, hipStream_t st) {
         else if (a.E <= 256) route_tails<4><<<nchunk, 64 * SPLIT_WAVES, lds, st>>>(a, tok);
         else route_tails<TOPK_MAX_J><<<nchunk, 64 * SPLIT_WAVES, lds, st>>>(a, tok);
         if (hipGetLastError() != hipSuccess) return MOE_ERR_LAUNCH;
-        return launch_group_place(a.S ? a.sidx : a.idx, n_all, E_all, tok * (a.k + a.S), nchunk, a.grp, a.P, a.P2, st);
+        return launch_group_place(a.S ? a.sidx : a.idx, n_all, E_all, tok * (a.k + a.S), nchunk, a.gsc.chunks, a.grp, a.P, a.P2, st);
     }
     size_t lds = 0;
     if (a.grp.counts) {
@@ -532,13 +532,14 @@ int launch_shared_route(const void* x, int xdt, const uint16_t* gate, int T, int
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
-int launch_group(const int32_t* idx, int n, int E, const GroupBufs& o, hipStream_t st, int P, int P2) {
+int launch_group(const int32_t* idx, int n, int E, const GroupBufs& o, const GroupScratch& sc, hipStream_t st, int P,
+                 int P2) {
     if ((o.items && (P < 1 || (P & (P - 1)))) || (o.items2 && (P2 < 1 || (P2 & (P2 - 1))))) return MOE_ERR_ARG;
     const int cs = group_chunk(n, 128), nchunk = (n + cs - 1) / cs;
-    if (group_split(n, E, nchunk, o)) {
-        k_group_count<<<nchunk, 256, (size_t)E * 4, st>>>(idx, n, E, cs, o.chunks);
+    if (group_split(n, E, nchunk, sc)) {
+        k_group_count<<<nchunk, 256, (size_t)E * 4, st>>>(idx, n, E, cs, sc.chunks);
         if (hipGetLastError() != hipSuccess) return MOE_ERR_LAUNCH;
-        return launch_group_place(idx, n, E, cs, nchunk, o, P, P2, st);
+        return launch_group_place(idx, n, E, cs, nchunk, sc.chunks, o, P, P2, st);
     }
     // one block: 16 waves (1024 threads) each placing a sixteenth of the slots from 1024 slots, else 4 waves; the
     // per-wave counts and the ids in LDS (at most 64 KB), else wave 0 places all of them

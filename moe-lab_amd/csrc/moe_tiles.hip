@@ -147,8 +147,8 @@ struct TileArgs {
     size_t plane;
     size_t eslot_off;      // dense int4 down: per-slot exponents (int32 [slots]) at this byte offset from the exponent bytes
     const int32_t* xexp;   // dense int4 gate/up: per-token exponents of x16 (actv) [T]
-    const uint8_t* xsum;   // dense int4 gate/up on exact weights: x16's group sums [T][ceil(K/128)][16 bytes]
     uint8_t* hterm;        // block-scaled MXFP4 gate/up: h leaves as 3-term records [T*k][ceil(N/128)] (no planes)
+    const uint8_t* xsum;   // dense int4 gate/up on exact weights: x16's group sums [T][ceil(K/128)][16 bytes]
 };
 
 // In-kernel grouping, one wave: pass y of the wave tiles' pass list (passes of P slots; an expert's slots in
@@ -1839,7 +1839,7 @@ int run_tiles_fmt(const ExpertsArgs& a) {
     if (a.stages & 1) {
         GroupBufs grp = a.grp;
         if (!two_lists) grp.items2 = nullptr;
-        int rc = ingroup || a.pregrouped ? 0 : launch_group(a.idx, nslots, w->E, grp, a.st, P_gu, P_dn);
+        int rc = ingroup || a.pregrouped ? 0 : launch_group(a.idx, nslots, w->E, grp, a.gsc, a.st, P_gu, P_dn);
         if (rc) return rc;
         TileArgs g = t;
         if (emit) {

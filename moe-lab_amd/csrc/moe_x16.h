@@ -56,9 +56,9 @@ __device__ __forceinline__ void x16_row(const void* __restrict__ x, int t, const
     uint4* out = reinterpret_cast<uint4*>(o.x16 + (size_t)t * d);
     const int nch = d >> 3;   // 8-element chunks, a multiple of 8
     constexpr int CPT = 4;    // chunks per lane and round (one round up to d = 2048)
-    float am = 0.f;
+    const bool one = nch <= 64 * CPT;   // the row stays in registers
+    float am = 0.f, v[CPT][8];
     for (int c0 = 0; c0 < nch; c0 += 64 * CPT) {
-        float v[CPT][8];
 #pragma unroll
         for (int i = 0; i < CPT; ++i)
             if (c0 + i * 64 + lane < nch) load_x8<XDT>(row, c0 + i * 64 + lane, v[i]);
@@ -73,11 +73,10 @@ __device__ __forceinline__ void x16_row(const void* __restrict__ x, int t, const
     int E = h16_exponent(amax);
     if (o.xsum && E == 0 && amax == amax) E = (int)((__float_as_uint(amax) >> 23) & 0xFFu) - 141;   // ordinary rows too
     if (lane == 0) o.xexp[t] = E;
-    for (int c0 = 0; c0 < nch; c0 += 64 * CPT) {   // the row again (cache hits)
-        float v[CPT][8];
+    for (int c0 = 0; c0 < nch; c0 += 64 * CPT) {   // longer rows: read again (cache hits)
 #pragma unroll
         for (int i = 0; i < CPT; ++i)
-            if (c0 + i * 64 + lane < nch) load_x8<XDT>(row, c0 + i * 64 + lane, v[i]);
+            if (!one && c0 + i * 64 + lane < nch) load_x8<XDT>(row, c0 + i * 64 + lane, v[i]);
 #pragma unroll
         for (int i = 0; i < CPT; ++i) {
             const int c = c0 + i * 64 + lane;
