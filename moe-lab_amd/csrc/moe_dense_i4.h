@@ -12,7 +12,7 @@
 // token n from LDS: piece p of token m lies at position p ^ (m & 15) of its 256-byte row, so the reads hit distinct banks.
 // The decode (11 VALU per word) and LDS reads of step j + 1 are placed between the MFMAs of step j
 // (sched_group_barrier); loads use buffer addressing (scalar base and slice offset, one 32-bit offset per lane: the 64-bit
-// address pairs of flat loads spilled). Both keep the wave's registers at 145 (M = 32: three blocks per CU) and 208.
+// address pairs of flat loads spilled). They take 167 (M = 32: three blocks per CU) and 209 registers.
 // Bound: decode and MFMA issue, then the chip's power: MFMAs alone on random data run at ~1.65 PFLOP/s here (1.6 GHz),
 // with 24 VALU per 128 MFMA cycles at ~1.5. Gate/up kernel, against the kernel before (16 x 16 tiles at 2 blocks per CU,
 // libm GLU, decode between whole steps): Mixtral T = 512 354 -> 294 us (820 TFLOP/s), Qwen3 T = 4096 320 -> 260.

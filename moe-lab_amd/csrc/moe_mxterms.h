@@ -11,10 +11,10 @@ template <int NTERM>
 __host__ __device__ constexpr int mx_rec() { return 16 * (8 * NTERM + 1); }
 
 // x rows (bf16) -> per (row, 128-input slice) records of REC = 16 (8 NTERM + 1) bytes: NTERM x 128 bytes of terms
-// at mx_pos (the records' code order, then the A operand's lane order), then the E8M0 byte of term t, block b at
+// in the records' code order, then the A operand's lane order (below), then the E8M0 byte of term t, block b at
 // 128 NTERM + 4 t + b. Inputs past K (K % 128 == 64) are zero codes with scale byte 127. This writes block i of
 // the rows' 4 ceil(K / 128) blocks each (nothing for i past them). h's records come from the gate/up epilogues
-// (mx_h_block).
+// (mx_h_terms).
 template <int NTERM>
 __device__ __forceinline__ void mx_terms_block(const uint16_t* __restrict__ src, int rows, int K,
                                                uint8_t* __restrict__ out, long i) {
