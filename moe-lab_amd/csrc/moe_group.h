@@ -199,14 +199,15 @@ __device__ void group_block(LD ld, int n, int E, const GroupBufs& o, int P, int 
 
 // ---------------------------------------------------------------------------- two-launch grouping of many slots
 // One workgroup groups n slots in time proportional to n, on one CU (n = 32768, E = 128, one placing wave: ~330 of the
-// 977 us of a Qwen3 T = 4096 layer, 654 us with this split). From GROUP_SPLIT_MIN slots the work is split over chunks of the slot list instead: the first launch counts each chunk's slots per expert
-// (chunks[c][E]: the router's tails do it as they write the ids, k_group_count otherwise), the second has one workgroup
-// per chunk (group_place), which sums the count rows itself (L2 hits, 64 KB at 128 chunks x 128 experts), so no
-// workgroup waits for another: the kernel boundary is the only hand-over. At most GROUP_MAX_CHUNKS chunks keep that
-// sum short at any n (256 chunks at Qwen3 T = 4096: placing 16.4 and tails 5.8 us, against 8.8 and 8.9). The line: layers with 1152 to 2048 slots run 0-2 us faster split than in one workgroup (OLMoE with
-// the router 79.7 -> 77.5 us at 1152 slots, 107.2 -> 106.1 at 2048; gpt-oss within 0.2 us), 3 us at 4096, 59-77 us from
-// 6144-8192; the calls below 1024 slots mostly group in-kernel (GW_MAXJ), and gpt-oss at 576-1024 slots shows no
-// difference.
+// 977 us of a Qwen3 T = 4096 layer, 654 us with this split). From GROUP_SPLIT_MIN slots the work is split over chunks of
+// the slot list instead: the first launch counts each chunk's slots per expert (chunks[c][E]: the router's tails do it as
+// they write the ids, k_group_count otherwise), the second has one workgroup per chunk (group_place), which sums the
+// count rows itself (L2 hits, 64 KB at 128 chunks x 128 experts), so no workgroup waits for another: the kernel
+// boundary is the only hand-over. At most GROUP_MAX_CHUNKS chunks keep that sum short at any n (256 chunks at Qwen3
+// T = 4096: placing 16.4 and tails 5.8 us, against 8.8 and 8.9). The line: layers with 1152 to 2048 slots run 0-2 us
+// faster split than in one workgroup (OLMoE with the router 79.7 -> 77.5 us at 1152 slots, 107.2 -> 106.1 at 2048;
+// gpt-oss within 0.2 us), 3 us at 4096, 59-77 us from 6144-8192; the calls below 1024 slots mostly group in-kernel
+// (GW_MAXJ), and gpt-oss at 576-1024 slots shows no difference.
 constexpr int GROUP_SPLIT_MIN = 1024;
 constexpr int GROUP_SPLIT_MAX_E = 2048;   // the placing workgroup's LDS: (GROUP_PW + 2) E ints
 constexpr int GROUP_MAX_CHUNKS = 128;

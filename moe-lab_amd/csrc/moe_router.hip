@@ -1,9 +1,10 @@
 // Router and slot grouping kernels for gfx950.
 //
 // router_logits: logits[t, e] = x[t] . Wr[e] (+ b[e]) in fp32, one wave per EPW experts x TPW tokens (router_logits_mm:
-// the same on the fp32 matrix cores for many tokens). route_finish, the next launch: the router tail (top-k, softmax) of one token per wave and, when the call asks for the grouping,
-// the sort of all T*k slots by expert (group_block) in its last workgroup to finish. At T = 1 the layer call skips
-// route_finish: the gate/up waves rank the token's logits themselves (moe_experts.hip).
+// the same on the fp32 matrix cores for many tokens). route_finish, the next launch: the router tail (top-k, softmax)
+// of one token per wave and, when the call asks for the grouping, the sort of all T*k slots by expert (group_block) in
+// its last workgroup to finish; with many slots route_tails only counts them and k_group_place sorts. At T = 1 the layer
+// call skips route_finish: the gate/up waves rank the token's logits themselves (moe_experts.hip).
 // The logit reduction order is fixed, so a CPU restatement reproduces every logit bit for bit and top-k ids
 // match exactly: lane l takes the 8-element chunks l, l+64, ... in order with fused multiply-adds in
 // element order, starting from +0; the 64 lane partials a[0..63] are combined by the DPP tree of
@@ -441,8 +442,8 @@ static int launch_group_place(const int32_t* idx, int n, int E, int cs, int nchu
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
-// logits (T > 1, fewer than ROUTER_MM_MIN logits: ROUTER_TPW tokens per wave share each loaded Wr chunk; T == 1: one expert per wave, fewer larger
-// waves or one wave per workgroup spread over E CUs measured no faster)
+// logits (T > 1, fewer than ROUTER_MM_MIN logits: ROUTER_TPW tokens per wave share each loaded Wr chunk; T == 1: one
+// expert per wave, fewer larger waves or one wave per workgroup spread over E CUs measured no faster)
 int launch_route_logits(const RouterArgs& a, hipStream_t st) {
     if ((long)a.T * a.lstride >= env_int("MOE_ROUTER_MM_MIN", ROUTER_MM_MIN) && a.d % 64 == 0) {
         const int nrb = (a.lstride + 15) / 16, n2 = (a.T + 31) / 32, n1 = (a.T + 15) / 16;
