@@ -536,8 +536,8 @@ int launch_shared_route(const void* x, int xdt, const uint16_t* gate, int T, int
 int launch_group(const int32_t* idx, int n, int E, const GroupBufs& o, const GroupScratch& sc, hipStream_t st, int P,
                  int P2) {
     if ((o.items && (P < 1 || (P & (P - 1)))) || (o.items2 && (P2 < 1 || (P2 & (P2 - 1))))) return MOE_ERR_ARG;
-    const int cs = group_chunk(n, 128), nchunk = (n + cs - 1) / cs;
-    if (group_split(n, E, nchunk, sc)) {
+    const int cs = n > 0 ? group_chunk(n, 128) : 128, nchunk = (n + cs - 1) / cs;   // no slots: no chunk
+    if (n > 0 && group_split(n, E, nchunk, sc)) {
         k_group_count<<<nchunk, 256, (size_t)E * 4, st>>>(idx, n, E, cs, sc.chunks);
         if (hipGetLastError() != hipSuccess) return MOE_ERR_LAUNCH;
         return launch_group_place(idx, n, E, cs, nchunk, sc.chunks, o, P, P2, st);

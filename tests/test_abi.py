@@ -3,6 +3,8 @@ invalid arguments before touching the GPU (host-side checks only; no kernel runs
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -83,6 +85,17 @@ def test_router_argument_errors():
     assert L.moe_router(p, p, None, 1, 2048, 128, 33, 1, 1.0, p, p, p, p, None) == -1   # k > 32
     assert L.moe_topk(p, 0, 1, 16, 17, 1, 1.0, p, p, None) == -1                        # k > E
     assert L.moe_group(p, 4, 0, p, p, p, p, p, None) == -1                              # E < 1
+
+
+def test_group_of_no_slots_returns():
+    """moe_group with n = 0 and no id or slot buffer is a valid call: it reaches its launch. In a process of its own, where
+    no GPU is visible (the launch then fails and says so), since a host fault would end the process."""
+    code = ("import ctypes, __graft_entry__ as g; g.load_package(); from moelab_amd import _lib; p = ctypes.c_void_p(4096); "
+            "print(_lib.lib().moe_group(None, 0, 8, p, p, None, p, p, None))")
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, env=env, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stderr[-500:])
+    assert int(r.stdout) == -4   # MOE_ERR_LAUNCH
 
 
 def test_router_group_and_layer_argument_errors():

@@ -114,6 +114,15 @@ def test_group_bit_exact(T, k, E, routing):
     assert (active.cpu().numpy()[len(a):] == -1).all()
 
 
+@pytest.mark.parametrize("E", [1, 8, 130])
+def test_group_of_no_slots(E):
+    from moelab_amd import router
+    counts, offsets, srt, active, meta = router.group(torch.empty((0, 4), dtype=torch.int32, device=DEV), E)
+    assert srt.numel() == 0 and meta.cpu().tolist() == [0, 0]
+    assert counts.cpu().tolist() == [0] * E and offsets.cpu().tolist() == [0] * (E + 1)
+    assert active.cpu().tolist() == [-1] * E
+
+
 def test_group_rejects_out_of_range_ids():
     from moelab_amd import router
     idx = torch.tensor([[0, 5], [3, 99], [-1, 3]], dtype=torch.int32, device=DEV)
