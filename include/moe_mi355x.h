@@ -178,9 +178,11 @@ int moe_group(const int32_t* idx, int n, int E, int32_t* counts, int32_t* offset
  *   exponent per row (no overflow and no flush to zero whatever a row's absolute scale); within a row, weights
  *   more than 2^13 below the row's largest |16 s|, |b| fall into fp16's subnormal range (absolute step 2^-19 of
  *   the row's largest |s|, |b|); ~1e-3 of the outputs' RMS in the worst case measured, 1.4e-3 with one scale
- *   group per row at 256x the others' (numpy emulation). From 21 to 32 slots per expert the gate/up (bf16 or
- *   fp16 x) also runs on fp16 MFMA, on the exact weights s (q - 8) and x in that fp16 form, with b + 8 s applied
- *   to the group sums of x: its error against 64 bits is that of the kernels at fewer slots.
+ *   group per row at 256x the others' (numpy emulation). From 17 to 32 slots per expert the down does the
+ *   same where its grid fills the chip (row blocks of 128 x passes of 128 slots >= 256), else both stages stay on exact
+ *   codes. Before such a down, from 21 slots per expert, the gate/up (bf16 or fp16 x) also runs on fp16 MFMA, on the
+ *   exact weights s (q - 8) and x in that fp16 form, with b + 8 s applied to the group sums of x: the call's error
+ *   against 64 bits is that of the exact-code gate/up before the same down.
  *   Requirements: d % 64 == 0, F % 64 == 0, F <= 16384; x, y, rows 16-byte aligned.
  *   workspace: moe_experts_workspace_bytes(...) bytes (any contents; every call writes what it reads). Calls
  *   sharing a workspace must be stream-ordered.

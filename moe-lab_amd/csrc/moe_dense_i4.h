@@ -22,7 +22,8 @@
 // row scaling: to 2^-22 of the row's largest), and what is left, sum over groups of (b + 8 s) XS with XS = the group's sum of
 // activations, is a product over groups of its own: one MFMA per GS = 4 (M = 16) or 2 slices and tile pair, lane group
 // g holding slice GS i + g, both factors as fp16 hi + lo (hi hi + lo hi + hi lo, 22 bits). k_x16 writes XS in A-operand form.
-// Against 64 bits the layer is then as far off as with the wave tiles (the fp16 rounding of h).
+// Used where the down takes the dense tiles anyway (make_plan): against 64 bits the layer is then as far off as with the wave
+// tiles' gate/up before the same down (2.08e-4 of the norm either way, fp32 outputs: the fp16 rounding of h and W_down).
 template <int NPROJ, int RT, int M, int BM, int MINB, bool EX = false>
 __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__   // buffer resources exist in device code only

@@ -1735,7 +1735,9 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
     constexpr int DP = 64;   // the dense tiles' pass
     constexpr int BN_GU = dense_bn<FMT, 2>(), BN_DN = dense_bn<FMT, 1>();
     const long dblocks = (long)((w->F + BN_GU - 1) / BN_GU) * max_passes(nslots, w->E, DP);
-    const long dn_blocks = (long)((w->d + BN_DN - 1) / BN_DN) * max_passes(nslots, w->E, DP);
+    // the dense down's line (dn_own below) was drawn in 128-token passes, and is kept there: calls under it keep the exact
+    // wave down
+    const long dn_blocks = (long)((w->d + BN_DN - 1) / BN_DN) * max_passes(nslots, w->E, 128);
     // MXFP4 with bf16 x: the block-scaled MFMA kernels (MOE_MXMFMA=0: the bf16-MFMA tiles). x's terms go to the x-planes
     // region, h's terms to the yp planes the split down would use; both must fit there, with 32-bit record offsets
     const size_t mx_xb = (size_t)T * ((w->d + 127) / 128) * mx_rec<2>();
@@ -1757,16 +1759,18 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
     const bool dense_gu_x = INT4 ? x_dtype != MOE_DTYPE_F32 : nx == 1;
     p.dense_gu = dense_gu_x && p.tiled && avg > min_avg &&
                  (dmode == 1 || (dmode < 0 && dblocks >= MOE_DENSE_MIN_BLOCKS));
-    // int4 up to the dense gate/up's line: the dense gate/up on exact weights (the wave tiles' codes are exact there, and the
-    // down's operands are fp16 already), 32-token passes at four blocks per CU, from 21 slots per expert. Layers, wave /
+    // int4 below the dense gate/up's line: whether the down takes the dense tiles (weights and h in fp16) by itself
+    const bool dn_own = INT4 && p.tiled && dmode != 0 && avg > dn_min_avg && (dmode == 1 || dn_blocks >= MOE_DENSE_MIN_BLOCKS);
+    // There, up to the dense gate/up's line: the dense gate/up on exact weights (the wave tiles' codes are exact too, and the
+    // down's operands are fp16 either way; where the down stays on the wave tiles, exact with h in two planes, so does the
+    // gate/up: the dense one writes h16 only), 32-token passes at four blocks per CU, from 21 slots per expert. Layers, wave /
     // exact dense: DeepSeek-V2-Lite T = 237 (29 slots) 141.4 / 128.3 us, Zipf 141.8 / 126.5; OLMoE T = 200 (25) 102.0 / 98.4,
     // Zipf 109.5 / 101.8, T = 256 (32) 114.6 / 102.9; Mixtral T = 120 (30) 266 / 240; Qwen3-235B T = 300 (19) 370 / 347; but
     // OLMoE T = 140 (18) 84.3 / 86.3, Qwen3 T = 300 (19) 120.9 / 121.5
-    p.i4_ex = INT4 && !p.dense_gu && dense_gu_x && p.tiled && avg > env_int("MOE_DENSE_EX_MIN_AVG", 20) && avg <= 32 &&
-              (dmode == 1 || (dmode < 0 && dblocks >= MOE_DENSE_MIN_BLOCKS));
+    p.i4_ex = dn_own && !p.dense_gu && dense_gu_x && avg > env_int("MOE_DENSE_EX_MIN_AVG", 20) && avg <= 32 &&
+              (dmode == 1 || dblocks >= MOE_DENSE_MIN_BLOCKS);
     p.dense_gu |= p.i4_ex;
-    p.dense_dn = p.dense_gu || (INT4 && p.tiled && dmode != 0 && avg > dn_min_avg &&
-                                (dmode == 1 || dn_blocks >= MOE_DENSE_MIN_BLOCKS));
+    p.dense_dn = p.dense_gu || dn_own;
     p.mxd = mx_fit && p.dense_gu && w->F % 32 == 0 && w->d % 64 == 0;
     p.wave_gu = p.tiled && !p.dense_gu && (avg <= 32 || dmode != 0);
     p.wave_dn = p.tiled && !p.dense_dn && (avg <= 32 || dmode != 0);

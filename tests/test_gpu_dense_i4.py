@@ -136,3 +136,25 @@ def test_router_writes_the_fp16_rows(T, E, k, d, monkeypatch):
     i2, w2 = router.route(x, wr, k)
     assert torch.equal(idx, i2) and torch.equal(wts, w2)
     assert torch.equal(y, experts.run_experts(s, x, idx, wts, out_dtype=torch.float32))
+
+
+@pytest.mark.parametrize("d,F,E,T,k", [(512, 1024, 32, 400, 2),    # gate/up blocks for the chip, 25 slots per expert
+                                       (1024, 64, 24, 480, 1),     # at the edge: 224 down blocks in 128-token passes, 256 in 64
+                                       (64, 8192, 8, 88, 2)])
+def test_exact_down_where_its_grid_is_small(monkeypatch, d, F, E, T, k):
+    """17 to 32 slots per expert and a down projection of few blocks: both stages stay on exact codes and two planes of h,
+    whatever the gate/up's grid. h = hi + lo keeps 2^-17 per term, so 1e-4 of the RMS is above 10 standard errors; the fp16
+    weights and h of the dense down (2^-12 per operand) miss it by ten times."""
+    from moelab_amd import _lib, experts
+    from moelab_amd.problem import baseline_int4_layer
+    from moelab_amd.shapes import MoEShape
+    monkeypatch.delenv("MOE_DENSE", raising=False)
+    assert 16 < (T * k + E - 1) // E <= 32
+    s = baseline_int4_layer(MoEShape("t", d=d, f=F, E=E, k=k), seed=d + T, device=DEV, router=False)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn((T, d), generator=g, device=DEV).to(torch.bfloat16)
+    idx = torch.rand((T, E), generator=g, device=DEV).topk(k, dim=1).indices.to(torch.int32)
+    wts = torch.rand((T, k), generator=g, device=DEV)
+    print(f"case small down d={d} F={F} E={E} T={T} k={k}", flush=True)
+    y = experts.run_experts(s, x, idx, wts, path=_lib.PATH_GROUPED, out_dtype=torch.float32)
+    assert_close(y, oracle_y(s, x, idx, wts), tol=1e-4, what=(d, F, E, T, k))
