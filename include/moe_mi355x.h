@@ -185,7 +185,8 @@ int moe_group(const int32_t* idx, int n, int E, int32_t* counts, int32_t* offset
  *   against 64 bits is that of the exact-code gate/up before the same down.
  *   Requirements: d % 64 == 0, F % 64 == 0, F <= 16384; x, y, rows 16-byte aligned.
  *   workspace: moe_experts_workspace_bytes(...) bytes (any contents; every call writes what it reads). Calls
- *   sharing a workspace must be stream-ordered.
+ *   sharing a workspace must be stream-ordered. With the tile-major copies a grouped call whose x (T d 2 bytes) or h
+ *   (T k F 2 bytes) passes 2^32 - 4096 bytes runs as equal blocks of tokens, each with a part of the workspace.
  */
 int moe_experts_run(const moe_experts_t* w, const void* x, int x_dtype, const int32_t* idx, const float* wts, int T,
                     int k, int act, int path, int nored, void* y, int y_dtype, const void* residual, void* workspace,

@@ -86,6 +86,27 @@ Layout layout(const moe_experts_t* w, int T, int k, int path) {
     return L;
 }
 
+// Tokens per block of a call (T: one block). The kernels on the tile-major copies address a block's rows of x (as bf16, fp16 or
+// MXFP4 term records) and h by 32-bit byte offsets under ACT_BYTES_MAX, so a grouped call with more than that runs as equal
+// blocks of tokens, one after another, each in its own part of the workspace (the two stages may be separate calls).
+int token_block(const moe_experts_t* w, int T, int k, int path) {
+    if (T < 1 || w->d < 1 || w->F < 1 || resolve_path(path, T) != MOE_PATH_GROUPED) return T;
+    if (!w->gate.tiles || !w->up.tiles || !w->down.tiles) return T;   // the row tiles take 64-bit offsets
+    size_t row = 2 * (size_t)k * w->F;   // of h
+    const size_t x = w->fmt == MOE_FMT_MXFP4 ? (size_t)((w->d + 127) / 128) * moe::MX_X_RECORD : 2 * (size_t)w->d;
+    if (row < x) row = x;
+    const size_t fit = row < moe::ACT_BYTES_MAX ? moe::ACT_BYTES_MAX / row : 1;
+    if ((size_t)T <= fit) return T;
+    const int nb = (int)((T + fit - 1) / fit);
+    return (T + nb - 1) / nb;
+}
+
+// the experts' part of a workspace
+size_t experts_bytes(const moe_experts_t* w, int T, int k, int path) {
+    const int Tb = token_block(w, T, k, path);
+    return Tb == T ? layout(w, T, k, path).total : layout(w, Tb, k, MOE_PATH_GROUPED).total * ((T + Tb - 1) / Tb);
+}
+
 int check_proj(const moe_proj_t& p) {
     if (!p.rows) return MOE_ERR_ARG;
     if (!aligned16(p.rows) || (p.tiles && !aligned16(p.tiles))) return MOE_ERR_ALIGN;
@@ -182,13 +203,13 @@ int moe_group(const int32_t* idx, int n, int E, int32_t* counts, int32_t* offset
 
 size_t moe_experts_workspace_bytes(const moe_experts_t* w, int T, int k, int path) {
     if (!w || T < 0 || k < 1) return 0;
-    return layout(w, T, k, path).total;
+    return experts_bytes(w, T, k, path);
 }
 
 size_t moe_shared_experts_workspace_bytes(const moe_experts_t* ws, int T) {
     if (!ws || T < 0 || ws->E < 1) return 0;
     const size_t n = (size_t)T * ws->E;
-    return layout(ws, T, ws->E, MOE_PATH_AUTO).total + 2 * align_up(n * 4);
+    return experts_bytes(ws, T, ws->E, MOE_PATH_AUTO) + 2 * align_up(n * 4);
 }
 
 int moe_shared_experts_run(const moe_experts_t* ws, const void* x, int x_dtype, int T, int act, const void* gate,
@@ -201,7 +222,7 @@ int moe_shared_experts_run(const moe_experts_t* ws, const void* x, int x_dtype, 
     if (!x || !y || !workspace) return x && y ? MOE_ERR_WORKSPACE : MOE_ERR_ARG;
     if (x_dtype < MOE_DTYPE_BF16 || x_dtype > MOE_DTYPE_F32) return MOE_ERR_DTYPE;
     if (!aligned16(x) || (gate && !aligned16(gate)) || !aligned16(workspace)) return MOE_ERR_ALIGN;
-    const size_t base = layout(ws, T, ws->E, MOE_PATH_AUTO).total;
+    const size_t base = experts_bytes(ws, T, ws->E, MOE_PATH_AUTO);
     if (workspace_bytes < moe_shared_experts_workspace_bytes(ws, T)) return MOE_ERR_WORKSPACE;
     const size_t n = (size_t)T * ws->E;
     int32_t* idx = (int32_t*)((char*)workspace + base);
@@ -215,7 +236,7 @@ int moe_shared_experts_run(const moe_experts_t* ws, const void* x, int x_dtype, 
 size_t moe_experts_shared_workspace_bytes(const moe_experts_t* w, int S, int T, int k, int path) {
     if (!w || T < 0 || k < 1 || S < 1 || k + S > 64) return 0;
     const size_t n = (size_t)T * (k + S);
-    return layout(w, T, k + S, path).total + 2 * align_up(n * 4);
+    return experts_bytes(w, T, k + S, path) + 2 * align_up(n * 4);
 }
 
 // routed + shared in one call: the slot lists [T, k + S] (routed ids outside [0, E - S) become -1, so they join no
@@ -233,7 +254,7 @@ int moe_experts_run_shared(const moe_experts_t* w, int S, const void* x, int x_d
     if (x_dtype < MOE_DTYPE_BF16 || x_dtype > MOE_DTYPE_F32) return MOE_ERR_DTYPE;
     if (!aligned16(x) || (gate && !aligned16(gate)) || !aligned16(workspace)) return MOE_ERR_ALIGN;
     if (workspace_bytes < moe_experts_shared_workspace_bytes(w, S, T, k, path)) return MOE_ERR_WORKSPACE;
-    const size_t base = layout(w, T, k + S, path).total;
+    const size_t base = experts_bytes(w, T, k + S, path);
     const size_t n = (size_t)T * (k + S);
     int32_t* idx2 = (int32_t*)((char*)workspace + base);
     float* wts2 = (float*)((char*)workspace + base + align_up(n * 4));
@@ -276,14 +297,14 @@ int layer_call(const moe_experts_t* w, int S, const void* x, int x_dtype, const 
 
 size_t moe_layer_workspace_bytes(const moe_experts_t* w, int T, int k) {
     if (!w || T < 0 || k < 1 || w->E < 1) return 0;
-    return layout(w, T, k, MOE_PATH_AUTO).total + align_up((size_t)T * w->E * 4);   // + the router logits
+    return experts_bytes(w, T, k, MOE_PATH_AUTO) + align_up((size_t)T * w->E * 4);   // + the router logits
 }
 
 size_t moe_layer_shared_workspace_bytes(const moe_experts_t* w, int S, int T, int k) {
     if (!w || T < 0 || k < 1 || S < 1 || S >= w->E || k + S > 64) return 0;
     const size_t n = (size_t)T * (k + S);
     // the experts' workspace for k + S slots, the router logits with the gate row, the merged slot lists
-    return layout(w, T, k + S, MOE_PATH_AUTO).total + align_up((size_t)T * (w->E - S + 1) * 4) + 2 * align_up(n * 4);
+    return experts_bytes(w, T, k + S, MOE_PATH_AUTO) + align_up((size_t)T * (w->E - S + 1) * 4) + 2 * align_up(n * 4);
 }
 
 int moe_layer_run(const moe_experts_t* w, const void* x, int x_dtype, const void* wr, const float* wr_bias, int T,
@@ -327,10 +348,23 @@ int experts_call(const moe_experts_t* w, const void* x, int x_dtype, const int32
     if (T == 0) return MOE_OK;
     if (!x || !idx || !wts || !y) return MOE_ERR_ARG;
     if (!aligned16(x) || !aligned16(y) || (residual && !aligned16(residual))) return MOE_ERR_ALIGN;
-    const Layout L = layout(w, T, k, path);
-    if (!workspace || workspace_bytes < L.total) return MOE_ERR_WORKSPACE;
+    const int Tb = token_block(w, T, k, path);
+    if (!workspace || workspace_bytes < experts_bytes(w, T, k, path)) return MOE_ERR_WORKSPACE;
     if (!aligned16(workspace)) return MOE_ERR_ALIGN;
     char* ws = (char*)workspace;
+    if (Tb < T) {
+        const size_t part = layout(w, Tb, k, MOE_PATH_GROUPED).total;
+        const size_t xrow = (size_t)w->d * (x_dtype == MOE_DTYPE_F32 ? 4 : 2), yrow = (size_t)w->d * (y_dtype == MOE_DTYPE_F32 ? 4 : 2);
+        for (int t0 = 0; t0 < T; t0 += Tb, ws += part) {
+            const size_t t = t0;
+            rc = experts_call(w, (const char*)x + t * xrow, x_dtype, idx + t * k, wts + t * k, T - t0 < Tb ? T - t0 : Tb, k, act,
+                              MOE_PATH_GROUPED, 0, (char*)y + t * yrow, y_dtype,
+                              residual ? (const char*)residual + t * yrow : nullptr, ws, part, stages, stream, nullptr, 1, 1.f);
+            if (rc) return rc;
+        }
+        return MOE_OK;
+    }
+    const Layout L = layout(w, T, k, path);
     moe::ExpertsArgs a{};
     a.w = w;
     a.x = x;
@@ -414,17 +448,19 @@ int layer_call(const moe_experts_t* w, int S, const void* x, int x_dtype, const 
     if (!aligned16(workspace)) return MOE_ERR_ALIGN;
     const int ks = k + S;   // slots per token
     const Layout L = layout(w, T, ks, MOE_PATH_AUTO);
+    const size_t base = experts_bytes(w, T, ks, MOE_PATH_AUTO);
+    const bool whole = token_block(w, T, ks, MOE_PATH_AUTO) == T;
     char* ws = (char*)workspace;
     hipStream_t st = (hipStream_t)stream;
     moe::RouterArgs ra{};
     ra.x = (const uint16_t*)x, ra.wr = (const uint16_t*)wr, ra.bias = wr_bias, ra.gate = (const uint16_t*)gate;
     ra.T = T, ra.d = w->d, ra.E = Er, ra.k = k, ra.norm = norm, ra.scale = scale;
-    ra.logits = (float*)(ws + L.total), ra.lstride = Er + (gate ? 1 : 0);
+    ra.logits = (float*)(ws + base), ra.lstride = Er + (gate ? 1 : 0);
     ra.idx = idx, ra.wts = wts, ra.S = S;
     const int32_t* eidx = idx;   // the slot lists the experts read
     const float* ewts = wts;
     if (S) {
-        ra.sidx = (int32_t*)(ws + L.total + align_up((size_t)T * (Er + 1) * 4));
+        ra.sidx = (int32_t*)(ws + base + align_up((size_t)T * (Er + 1) * 4));
         ra.swts = (float*)((char*)ra.sidx + align_up((size_t)T * ks * 4));
         eidx = ra.sidx, ewts = ra.swts;
     }
@@ -432,10 +468,10 @@ int layer_call(const moe_experts_t* w, int S, const void* x, int x_dtype, const 
         rc = moe::launch_route(ra, false, st);
         if (rc) return rc;
         return experts_call(w, x, x_dtype, idx, wts, T, k, act, MOE_PATH_AUTO, 0, y, y_dtype, residual, workspace,
-                            L.total, MOE_STAGE_ALL, stream, ra.logits, norm, scale);
+                            base, MOE_STAGE_ALL, stream, ra.logits, norm, scale);
     }
     int pregrouped = 0, x_ready = 0;
-    if (resolve_path(MOE_PATH_AUTO, T) == MOE_PATH_GROUPED) {
+    if (whole && resolve_path(MOE_PATH_AUTO, T) == MOE_PATH_GROUPED) {   // (blocks of tokens are grouped by their own calls)
         const moe::TilePasses tp = moe::tile_passes(w, T, ks, x_dtype);
         if (tp.mx) {   // the block-scaled MXFP4 tiles: the finishing launch also writes x's term records
             ra.xterm = (uint8_t*)(ws + L.xp);
@@ -456,7 +492,7 @@ int layer_call(const moe_experts_t* w, int S, const void* x, int x_dtype, const 
     rc = moe::launch_route(ra, true, st);
     if (rc) return rc;
     return experts_call(w, x, x_dtype, eidx, ewts, T, ks, act, MOE_PATH_AUTO, 0, y, y_dtype, residual, workspace,
-                        L.total, MOE_STAGE_ALL, stream, nullptr, 1, 1.f, pregrouped, x_ready);
+                        base, MOE_STAGE_ALL, stream, nullptr, 1, 1.f, pregrouped, x_ready);
 }
 
 }  // namespace

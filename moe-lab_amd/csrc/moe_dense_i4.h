@@ -316,7 +316,7 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
             bg[h] = a.b0 ? a.b0[r] : 0.f;
             bu[h] = a.b1 ? a.b1[r] : 0.f;
         }
-        const __amdgpu_buffer_rsrc_t hb = buffer_of(a.hout, 0xFFFFF000u);   // a dead token's offset lies past it
+        const __amdgpu_buffer_rsrc_t hb = buffer_of(a.hout, (uint32_t)ACT_BYTES_MAX);   // a dead token's offset lies past it
         const bool odd = ln & 1;
         const uint32_t lofs = 2u * (uint32_t)(ln & ~1), psel = odd ? 0x05040100u : 0x01000504u;   // (own, received)
         each_quad([&](int t, int q, int j0, const int (&xe)[4], const int (&sl)[4]) __attribute__((always_inline)) {

@@ -75,6 +75,11 @@ int launch_topk(const void* logits, int dtype, int T, int E, int k, int norm, fl
 // P2 slots); with sc.chunks and many slots in two launches, else in one workgroup
 int launch_group(const int32_t* idx, int n, int E, const GroupBufs& o, const GroupScratch& sc, hipStream_t st, int P = 0,
                  int P2 = 0);
+// Bytes of one block's x (x16, planes, term records) or of one h plane that the kernels on the tile-major copies can address:
+// 32-bit offsets of 16-byte accesses through buffer descriptors, the last 4 KiB kept for the stores of dead tokens (dropped).
+// moe_api.hip splits larger calls into blocks of tokens.
+constexpr size_t ACT_BYTES_MAX = 0xFFFFF000u;
+constexpr size_t MX_X_RECORD = 272;   // bytes of x's term record per token and 128 inputs (mx_rec<2>)
 // tuning and test knobs from the environment, read per call
 inline int env_int(const char* name, int dflt) {
     const char* v = getenv(name);

@@ -3,12 +3,14 @@
 // finishing launch when a layer call feeds those tiles.
 #pragma once
 #include "moe_common.h"
+#include "moe_internal.h"
 
 namespace moe {
 
 // block-scaled MXFP4 tiles: bytes of one (activation row, 128-input slice) record of NTERM fp8 terms + scales
 template <int NTERM>
 __host__ __device__ constexpr int mx_rec() { return 16 * (8 * NTERM + 1); }
+static_assert(mx_rec<2>() == MX_X_RECORD, "the size the blocks of tokens are taken from");
 
 // x rows (bf16) -> per (row, 128-input slice) records of REC = 16 (8 NTERM + 1) bytes: NTERM x 128 bytes of terms
 // in the records' code order, then the A operand's lane order (below), then the E8M0 byte of term t, block b at

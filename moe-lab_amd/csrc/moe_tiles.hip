@@ -1739,7 +1739,8 @@ Plan make_plan(const moe_experts_t* w, int T, int k, int x_dtype) {
     // wave down
     const long dn_blocks = (long)((w->d + BN_DN - 1) / BN_DN) * max_passes(nslots, w->E, 128);
     // MXFP4 with bf16 x: the block-scaled MFMA kernels (MOE_MXMFMA=0: the bf16-MFMA tiles). x's terms go to the x-planes
-    // region, h's terms to the yp planes the split down would use; both must fit there, with 32-bit record offsets
+    // region, h's terms to the yp planes the split down would use; both must fit there, h's with 32-bit record offsets (x's
+    // have them in any block of tokens: ACT_BYTES_MAX)
     const size_t mx_xb = (size_t)T * ((w->d + 127) / 128) * mx_rec<2>();
     const size_t mx_hb = (size_t)nslots * ((w->F + 127) / 128) * mx_rec<3>();
     const bool mx_fit = !INT4 && nx == 1 && env_int("MOE_MXMFMA", 1) && mx_xb <= (size_t)6 * T * w->d &&

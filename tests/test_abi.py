@@ -50,6 +50,31 @@ def test_workspace_query_host_only():
     assert grouped >= 256 * 768 * 2 + 256 * 2048 * 4
 
 
+@pytest.mark.parametrize("fmt,E,d,F,k,fit", [
+    (0, 8, 4096, 14336, 2, (2 ** 32 - 4096) // (2 * 2 * 14336)),         # h: Mixtral, 74898 tokens
+    (0, 64, 2048, 1024, 8, (2 ** 32 - 4096) // (2 * 8 * 1024)),          # 2^32 bytes of h at T = 2^18
+    (0, 8, 4096, 64, 1, (2 ** 32 - 4096) // (2 * 4096)),                 # x16
+    (1, 32, 4096, 64, 1, (2 ** 32 - 4096) // (32 * 272)),                # MXFP4: x's term records
+])
+def test_calls_past_32_bit_offsets_are_split(fmt, E, d, F, k, fit):
+    """The kernels on the tile-major copies address x and h with 32 bits: from the first token past that a call takes the
+    workspace of two equal blocks of tokens. Without the copies (64-bit kernels) it stays one piece."""
+    from moelab_amd import _lib
+    L = _lib.lib()
+    fake = ctypes.c_void_p(4096)
+    p = _lib.Proj(fake, None, fake)
+    w, rows = _lib.Experts(fmt, E, d, F, p, p, p), _desc(E=E, d=d, F=F, fmt=fmt)
+    size = lambda w, T, path=_lib.PATH_GROUPED: L.moe_experts_workspace_bytes(w, T, k, path)   # noqa: E731
+    assert size(w, fit) == size(rows, fit)
+    assert size(w, fit + 1) == 2 * size(w, fit // 2 + 1) != size(rows, fit + 1)
+    assert size(w, 3 * fit) == 3 * size(w, fit) and size(w, 3 * fit, _lib.PATH_AUTO) == size(w, 3 * fit)
+    assert size(w, 3 * fit, _lib.PATH_SLOTS) == size(rows, 3 * fit, _lib.PATH_SLOTS)
+    # the calls that add their own parts, and the check before any launch
+    assert L.moe_layer_workspace_bytes(w, fit + 1, k) >= size(w, fit + 1) + 4 * E * (fit + 1)
+    ws = ctypes.c_void_p(8192)
+    assert L.moe_experts_run(w, fake, 0, fake, fake, fit + 1, k, 0, 0, 0, fake, 0, None, ws, size(w, fit + 1) - 1, None) == -3
+
+
 @pytest.mark.parametrize("case,rc", [("d_not_64", -1), ("bad_fmt", -2), ("bad_act", -1), ("no_ws", -3),
                                      ("bad_dtype", -2), ("nored_grouped", -1), ("misaligned", -5)])
 def test_argument_errors_before_launch(case, rc):
