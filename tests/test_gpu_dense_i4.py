@@ -37,23 +37,28 @@ def test_token_tile_edges(monkeypatch, counts, d, F, act, dtype):
     _run(d, F, counts, act, dtype, seed=sum(counts) + d)
 
 
-def test_dead_tokens_and_large_h_write_only_their_slots(monkeypatch):
-    """h beyond fp16 (per-chunk exponents, the epilogue's scaled branch) beside ordinary tokens in one pass."""
+def test_large_and_small_h_beside_ordinary_tokens(monkeypatch):
+    """h beyond fp16 and below 2^-8 (per-chunk exponents, the epilogue's scaled branch) beside ordinary tokens in one pass, in
+    passes with dead tokens (100 and 50 slots): every row against its class's own size, so that no row takes another's
+    exponent or values. (Dead tokens repeat the expert's last slot: what they would store is that slot's own row.)"""
     from moelab_amd import _lib, experts
     from moelab_amd.problem import baseline_int4_layer
     from moelab_amd.shapes import MoEShape
     monkeypatch.setenv("MOE_DENSE", "1")
     d, F, E, T = 256, 192, 2, 150
     s = baseline_int4_layer(MoEShape("t", d=d, f=F, E=E, k=1), seed=9, device=DEV, router=False)
-    x = torch.randn((T, d), device=DEV).to(torch.bfloat16)
+    x = torch.randn((T, d), generator=torch.Generator(device=DEV).manual_seed(9), device=DEV).to(torch.bfloat16)
     x[::7] *= 3e3      # |h| to ~1e8
     x[3::7] *= 1e-3    # chunks below 2^-8
     idx = (torch.arange(T, device=DEV, dtype=torch.int32) % 3 == 0).to(torch.int32)[:, None].contiguous()
     wts = torch.ones((T, 1), device=DEV)
     y = experts.run_experts(s, x, idx, wts, path=_lib.PATH_GROUPED, out_dtype=torch.float32)
     want = oracle_y(s, x, idx, wts)
-    for rows in (slice(0, None, 7), slice(3, None, 7), slice(1, None, 7)):
-        assert_close(y[rows], want[rows], tol=1e-2, what=rows)
+    for r in range(7):
+        assert_close(y[r::7], want[r::7], tol=1e-2, what=r)
+    # row by row too, in norms (fp16 operands: 2^-12 each, about 3.5e-4 of the norm)
+    off = np.linalg.norm(y.cpu().numpy() - want, axis=1) / np.linalg.norm(want, axis=1)
+    assert off.max() < 2e-3, (int(off.argmax()), float(off.max()))
 
 
 @pytest.mark.parametrize("F", [64, 192, 1088, 4096])   # 4096: a wave per slot
