@@ -1,8 +1,8 @@
 // int4 dense tiles on fp16 MFMA (included by moe_tiles.hip after TileArgs): calls with many tokens per expert.
 #pragma once
 
-// A 4-wave block owns 128 RT rows of one expert (per projection) and one pass of up to BM of its tokens, NT tiles of M;
-// wave w takes 32 RT of the rows for all the pass's tokens, so each weight is decoded once per pass. Per 128-input slice
+// A 4-wave block owns 128 rows of one expert (per projection) and one pass of up to BM of its tokens, NT tiles of M;
+// wave w takes 32 of the rows for all the pass's tokens, so each weight is decoded once per pass. Per 128-input slice
 // the tokens' activations (x16 / h16, fp16) come into LDS by DMA and the wave's weight records into registers, both one
 // slice ahead in two buffers; one wait and one barrier per slice.
 // Token-major product D[token, row]: A = activations, B = weights. M = 32: v_mfma_f32_32x32x16_f16, 8 steps of 16 inputs
@@ -20,19 +20,17 @@
 // EX (gate/up): products on exact weights, for loads where the wave tiles' exact codes were used before. The decode
 // takes s (q - 8) instead of s q + b: 8 + 3 significant bits, which fp16 holds exactly (below the subnormal line of the
 // row scaling: to 2^-22 of the row's largest), and what is left, sum over groups of (b + 8 s) XS with XS = the group's sum of
-// activations, is a product over groups of its own: one MFMA per GS = 4 (M = 16) or 2 slices and tile pair, lane group
-// g holding slice GS i + g, both factors as fp16 hi + lo (hi hi + lo hi + hi lo, 22 bits). k_x16 writes XS in A-operand form.
+// activations, is a product over groups of its own: one MFMA (M = 32) per two slices and tile pair, lane group g holding
+// slice 2 i + g, both factors as fp16 hi + lo (hi hi + lo hi + hi lo, 22 bits). k_x16 writes XS in A-operand form.
 // Used where the down takes the dense tiles anyway (make_plan): against 64 bits the layer is then as far off as with the wave
 // tiles' gate/up before the same down (2.08e-4 of the norm either way, fp32 outputs: the fp16 rounding of h and W_down).
-template <int NPROJ, int RT, int M, int BM, int MINB, bool EX = false>
+template <int NPROJ, int M, int BM, int MINB, bool EX = false>
 __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
 #ifdef __HIP_DEVICE_COMPILE__   // buffer resources exist in device code only
-    static_assert(!EX || NPROJ == 2, "exact weights: gate/up");
-    constexpr int NT = BM / M, BN = 128 * RT;
-    constexpr int GS = 64 / M;            // EX: slices per MFMA of the group-sum term
-    constexpr int CT = NPROJ * RT;        // 32-row groups per wave
-    constexpr int H = 32 / M;             // B tiles per group
-    constexpr int CB = CT * H;
+    static_assert(!EX || (NPROJ == 2 && M == 32), "exact weights: gate/up in tiles of 32 tokens");
+    constexpr int NT = BM / M, BN = 128;
+    constexpr int H = 32 / M;             // B tiles per projection: the wave's 32 rows
+    constexpr int CB = NPROJ * H;
     constexpr int NJ = M / 4;             // steps per slice
     constexpr int NQ = M == 32 ? 4 : 1;   // groups of 4 tokens per accumulator
     constexpr int SB = TILE_SLICE_INT4;
@@ -69,27 +67,25 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
     const int per = (nsl + a.ksplit - 1) / a.ksplit;
     const int sb0 = ks * per;                                // this block's slices: sb0 .. sb0 + scnt - 1
     const int scnt = nsl - sb0 < per ? nsl - sb0 : per;   // >= 1 (the host splits only when it is)
-    const int r0 = rb * BN + wave * 32 * RT;
-    const bool wvalid = r0 < N;           // N % (32 RT) == 0: a wave's rows are all in range or all out
+    const int r0 = rb * BN + wave * 32;
+    const bool wvalid = r0 < N;           // N % 32 == 0: a wave's rows are all in range or all out
     const uint32_t trec = (uint32_t)nsl * SB;   // one 16-row tile's records
-    __amdgpu_buffer_rsrc_t wb[NPROJ];     // the wave's 2 RT row tiles of each projection, consecutive
+    __amdgpu_buffer_rsrc_t wb[NPROJ];     // the wave's two row tiles of each projection, consecutive
 #pragma unroll
     for (int p = 0; p < NPROJ; ++p)
-        wb[p] = buffer_of((p ? a.W1 : a.W0) + ((size_t)e * (N >> 4) + (wvalid ? (r0 >> 4) : 0)) * (size_t)trec, 2u * RT * trec);
+        wb[p] = buffer_of((p ? a.W1 : a.W0) + ((size_t)e * (N >> 4) + (wvalid ? (r0 >> 4) : 0)) * (size_t)trec, 2u * trec);
     const uint32_t wofs = M == 32 ? (uint32_t)(ln >> 4) * trec + 16u * (ln & 15) + 512u * lg : 16u * lane;
     const uint32_t mofs = (M == 32 ? (uint32_t)(ln >> 4) * trec : 0u) + 1024u + 8u * (ln & 15);
-    struct WS { u32x4 q[CT][2]; u32x2 m[CB]; };
+    struct WS { u32x4 q[NPROJ][2]; u32x2 m[CB]; };
     auto fetch_w = [&](int s, WS& w) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < CT; ++c) {
-            const int so = 2 * (c % RT) * (int)trec + s * SB;
+        for (int p = 0; p < NPROJ; ++p)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                w.q[c][h] = __builtin_amdgcn_raw_buffer_load_b128(wb[c / RT], wofs + (M == 32 ? 256 * h : 0),
-                                                                  so + (M == 32 ? 0 : h * (int)trec), 0);
-                if (h < H) w.m[c * H + h] = __builtin_amdgcn_raw_buffer_load_b64(wb[c / RT], mofs, so + h * (int)trec, 0);
+                w.q[p][h] = __builtin_amdgcn_raw_buffer_load_b128(wb[p], wofs + (M == 32 ? 256 * h : 0),
+                                                                  s * SB + (M == 32 ? 0 : h * (int)trec), 0);
+                if (h < H) w.m[p * H + h] = __builtin_amdgcn_raw_buffer_load_b64(wb[p], mofs, s * SB + h * (int)trec, 0);
             }
-        }
     };
     WS wa, wn;
     fetch_w(sb0, wa);                     // in flight while the pass's tokens are looked up
@@ -207,20 +203,18 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        // EX: the group-sum term of slices s4 .. s4 + GS - 1 (s4 = GS i), loaded at slice s4, multiplied two slices later
+        // EX: the group-sum term of slices s2 and s2 + 1 (s2 even), loaded at slice s2, multiplied two slices later
         f16x8 gx[EX ? L : 1];
         u32x2 gm[EX ? CB : 1];
-        auto fetch_g = [&](int s4) __attribute__((always_inline)) {
+        auto fetch_g = [&](int s2) __attribute__((always_inline)) {
             if constexpr (EX) {
-                const int sl = s4 + lg < nsl ? s4 + lg : nsl - 1;
+                const int sl = s2 + lg < nsl ? s2 + lg : nsl - 1;
 #pragma unroll
                 for (int t = 0; t < L; ++t)
                     gx[t] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(gb, grow[t] + 16u * sl, 0, 0));
 #pragma unroll
-                for (int b = 0; b < CB; ++b)
-                    gm[b] = __builtin_amdgcn_raw_buffer_load_b64(wb[b / (RT * H)], mofs + (uint32_t)(sl * SB),
-                                                                  (b % (RT * H)) * (2 / H) * (int)trec, 0);
-                if (s4 + lg >= nsl)
+                for (int b = 0; b < CB; ++b) gm[b] = __builtin_amdgcn_raw_buffer_load_b64(wb[b], mofs + (uint32_t)(sl * SB), 0, 0);
+                if (s2 + lg >= nsl)
 #pragma unroll
                     for (int b = 0; b < CB; ++b) gm[b] = u32x2{0u, 0u};
             }
@@ -238,10 +232,7 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
                     }
                     const f16x8 Bg = {hi[0], hi[1], lo[0], lo[1], hi[0], hi[1], (_Float16)0, (_Float16)0};
 #pragma unroll
-                    for (int t = 0; t < L; ++t) {
-                        if constexpr (M == 32) acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(gx[t], Bg, acc[b][t], 0, 0, 0);
-                        else acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(gx[t], Bg, acc[b][t], 0, 0, 0);
-                    }
+                    for (int t = 0; t < L; ++t) acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(gx[t], Bg, acc[b][t], 0, 0, 0);
                 }
             }
         };
@@ -253,8 +244,8 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
             fetch_w(sb0 + j + 1, wn);
             fetch_x(sb0 + j + 1, sX1);
             if constexpr (EX) {
-                if (GS == 4 ? (j & 2) : j) apply_g();
-                if (GS == 2 || !(j & 2)) fetch_g(j);
+                if (j) apply_g();
+                fetch_g(j);
             }
             compute(sX0, wa);
             MOE_VMWAIT0();
@@ -267,8 +258,8 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
             MOE_BARRIER();
         }
         if constexpr (EX) {   // the last group sums: fetched in the loop but not multiplied, or not fetched yet
-            if (GS == 4 ? (j & 2) : j) apply_g();
-            if ((GS == 2 || !(j & 2)) && j < scnt) {
+            if (j) apply_g();
+            if (j < scnt) {
                 fetch_g(j);
                 apply_g();
             }
@@ -289,7 +280,7 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
     int rex[CB];   // row exponents (the records hold s 2^-E, b 2^-E), plus the decode's
 #pragma unroll
     for (int b = 0; b < CB; ++b)
-        rex[b] = tile_row_exps(b / (RT * H) ? a.W1 : a.W0, a.E, N, K)[(size_t)e * N + r0 + M * (b % (RT * H)) + ln] + DEC_EXP;
+        rex[b] = tile_row_exps(b / H ? a.W1 : a.W0, a.E, N, K)[(size_t)e * N + r0 + M * (b % H) + ln] + DEC_EXP;
     auto each_quad = [&](auto fn) __attribute__((always_inline)) {   // fn(t, q, first token, exponents, slots) of 4 tokens
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -306,7 +297,6 @@ __global__ void __launch_bounds__(256, MINB) k_dense_i4(TileArgs a) {
     if constexpr (NPROJ == 2) {
         // h of the wave's 32 rows as fp16 h16 = h 2^-e, e per (slot, 32-row chunk): h16_exponent of the chunk's largest.
         // Two tokens' values of a lane pair are exchanged so that each lane stores two adjacent rows of one token.
-        static_assert(RT == 1, "one 32-row chunk of h per wave");
         int8_t* hexp_out = reinterpret_cast<int8_t*>(a.hout2);
         const int nch = N >> 5;
         float bg[H], bu[H];

@@ -1696,14 +1696,14 @@ int launch_dense(TileArgs t, int nslots, hipStream_t st) {
     k_dense<NPROJ><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
-template <int NPROJ, int RT, int M, int BM, int MINB, bool EX = false>
+template <int NPROJ, int M, int BM, int MINB, bool EX = false>
 int launch_dense_i4(TileArgs t, int nslots, hipStream_t st) {
-    constexpr int BN = 128 * RT;
-    if (t.N % (32 * RT)) return MOE_ERR_ARG;   // whole row tiles per wave
+    constexpr int BN = dense_bn<FmtInt4, NPROJ>();
+    if (t.N % 32) return MOE_ERR_ARG;   // whole row tiles per wave
     if (NPROJ == 2) t.ksplit = 1;
     const long nblk = ((long)((t.N + BN - 1) / BN) * max_passes(nslots, t.E, BM) * t.ksplit + 7) / 8 * 8;
     if (nblk > 0x7FFFFFF8L) return MOE_ERR_ARG;
-    k_dense_i4<NPROJ, RT, M, BM, MINB, EX><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
+    k_dense_i4<NPROJ, M, BM, MINB, EX><<<dim3((unsigned)nblk), 256, 0, st>>>(t);
     return hipGetLastError() == hipSuccess ? 0 : MOE_ERR_LAUNCH;
 }
 
@@ -1896,9 +1896,9 @@ int run_tiles_fmt(const ExpertsArgs& a) {
         } else if (mxd) rc = 0;
         else if (dense_gu) {
             if constexpr (!INT4) rc = launch_dense<2>(g, nslots, a.st);
-            else if (pl.i4_ex) rc = launch_dense_i4<2, 1, 32, 32, 4, true>(g, nslots, a.st);
-            else if (pl.i4_m == 16) rc = launch_dense_i4<2, 1, 16, 64, 2>(g, nslots, a.st);
-            else rc = launch_dense_i4<2, 1, 32, 64, 3>(g, nslots, a.st);
+            else if (pl.i4_ex) rc = launch_dense_i4<2, 32, 32, 4, true>(g, nslots, a.st);
+            else if (pl.i4_m == 16) rc = launch_dense_i4<2, 16, 64, 2>(g, nslots, a.st);
+            else rc = launch_dense_i4<2, 32, 64, 3>(g, nslots, a.st);
         }
         else if (wave_gu && h16)
             rc = launch_wave_tile<FMT, 2, MOE_WAVE_RT_GU, MOE_WAVE_D_GU, INT4>(g, nt, nslots, a.st, a.nx);
@@ -1951,7 +1951,7 @@ int run_tiles_fmt(const ExpertsArgs& a) {
         } else if (dense_dn) {
             // int4: 32 rows per wave at four blocks per CU; 64 rows (three blocks) or 32-token tiles measured slower on
             // every shape but Qwen3 T = 4096 (even)
-            if constexpr (INT4) rc = launch_dense_i4<1, 1, 16, 64, 4>(d, nslots, a.st);
+            if constexpr (INT4) rc = launch_dense_i4<1, 16, 64, 4>(d, nslots, a.st);
             else rc = launch_dense<1>(d, nslots, a.st);
         }
         else if (wave_dn && wide_dn(MOE_WAVE_RT_DN_WIDE))
