@@ -967,8 +967,9 @@ __global__ void __launch_bounds__(64) k_wave_tile(TileArgs a) {
 // ============================================================================ dense tiles (many tokens per expert)
 // Where an expert's token count makes the contraction dense (tens to hundreds of tokens per expert: prefill, the
 // shared experts), each block keeps its weight tiles for a pass of 64 tokens and multiplies them on MFMA against
-// activations staged once per block in LDS: k_dense_i4 (int4, moe_dense_i4.h), k_mxd (MXFP4 with bf16 x) and k_dense
-// (MXFP4 with fp16 / fp32 x, or MOE_MXMFMA=0: exact codes on bf16 MFMA).
+// activations staged once per block in LDS: k_dense_i4 (int4 with bf16 or fp16 x, moe_dense_i4.h), k_mxd (MXFP4 with bf16 x)
+// and k_dense (MXFP4 with bf16 x where k_mxd's records do not fit the workspace or MOE_MXMFMA=0: exact codes on bf16 MFMA).
+// fp32 x, and fp16 x on MXFP4, stay on the wave tiles at any size.
 #define MOE_LDSP(p) ((__attribute__((address_space(3))) void*)(p))
 // s_waitcnt vmcnt(0) with the other counters left alone (gfx9 encoding)
 #define MOE_VMWAIT0() __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8))
